@@ -492,3 +492,53 @@ def test_trsv_level_order_same_result(dev, name):
     assert np.array_equal(out[0], out[1])
     L, U, dinv = split_factors(rp, ci, lu, dpos)
     assert rel_err(out[1], oracle.upper_solve(U, dinv, oracle.lower_solve(L, b))) < 1e-12
+
+
+def _rows_of_lengths(lens, n, seed):
+    """CSR with the given row lengths (repeated), the diagonal among each row's
+    columns and dominant."""
+    rng = np.random.default_rng(seed)
+    rp, ci, v = [0], [], []
+    for i in range(n):
+        m = min(lens[i % len(lens)], n)
+        c = rng.choice(n - 1, m - 1, replace=False)
+        c = np.sort(np.append(np.where(c >= i, c + 1, c), i))
+        a = rng.uniform(-1, 1, m)
+        a[c == i] = 1.5 * np.abs(a).sum() + 1.0
+        ci.append(c)
+        v.append(a)
+        rp.append(rp[-1] + m)
+    return np.array(rp, np.int32), np.concatenate(ci).astype(np.int32), np.concatenate(v)
+
+
+@pytest.mark.parametrize("lens", [(1, 15, 16, 17), (16, 17, 63, 64, 65), (2, 2047, 3), (1500, 1, 1),
+                                  (17,)], ids=str)
+def test_csr_row_blocks_mixed_lengths(dev, lens):
+    """Rows at the edges of the lane / wave split of the LDS row blocks
+    (XS_CSR_ROW_LANE entries), FP64 products and epilogues and the FP32 inner
+    solve over the same blocks.  Bound: a row of m products summed in any order
+    is within m eps sum |a x| of the exact sum, and so is the oracle's."""
+    import torch
+    n = 2300 if max(lens) > 1000 else 1601
+    A = _rows_of_lengths(lens, n, 5)
+    say(f"[csr rows] lens={lens} n={n}")
+    rng = np.random.default_rng(4)
+    x, b = rng.uniform(-1, 1, n), rng.uniform(-1, 1, n)
+    bound = 2 * max(lens) * 2.3e-16 * (gen.spmv((A[0], A[1], np.abs(A[2])), np.abs(x)) + np.abs(b))
+    S = XSolver()
+    S.mat_setup(*A)
+    S.set_option("spmv_kernel", 0)
+    assert S.time_ms("spmv:kernel") == 0
+    yd = torch.empty(n, dtype=torch.float64, device=dev)
+    S.spmv(dev_tensor(x, dev), yd, torch_stream())
+    assert np.all(np.abs(yd.cpu().numpy() - oracle.spmv(A, x)) <= bound)
+    S.bmax(dev_tensor(b, dev), dev_tensor(x, dev), yd, torch_stream())
+    assert np.all(np.abs(yd.cpu().numpy() - oracle.bmax(A, b, x)) <= bound)
+    S.ksp_settype("bicgstab")
+    S.ksp_setoption(1e-10, 200)
+    S.pc_settype("jacobi")
+    for precision in (0, 1):
+        S.set_option("precision", precision)
+        xs, st = S.solve(b)
+        assert st == 0 and true_relres(A, b, xs) < 1e-10
+    S.close()

@@ -348,3 +348,64 @@ __device__ __forceinline__ void reduce_finish(double (&v)[NV], const xs_reduce &
     do_finish(R, t4, NV);
   }
 }
+
+// ---------------------------------------------------------------------------
+// LDS row blocks of the CSR SpMV (FP64 and FP32).  What bounded it: one
+// thread summed each row from LDS, and a block waited for its longest row --
+// a row of 2000 entries is a chain of 2000 LDS reads (262147 rows of 4 to
+// 2000 entries, 2.8e6 in all: 70 us, 0.55 TB/s).  Rows of more than
+// XS_CSR_ROW_LANE entries are summed by their wave instead.
+// ---------------------------------------------------------------------------
+#define XS_CSR_ROW_LANE 16
+// prod[k] = v[e0 + k] x[ci[e0 + k]], k < ne: four entries per thread and step,
+// their loads branch-free (past the end the last entry is read again) so that
+// all are issued before any wait
+template <class T>
+__device__ __forceinline__ void csr_stage(T *prod, int e0, int ne, const int *__restrict__ ci,
+                                          const T *__restrict__ v, const T *__restrict__ x) {
+  for (int k0 = threadIdx.x; k0 < ne; k0 += 4 * XS_BLOCK) {
+    int c[4];
+    T a[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int k = e0 + min(k0 + q * XS_BLOCK, ne - 1);
+      c[q] = ci[k];
+      a[q] = v[k];
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const T p = a[q] * x[c[q]];
+      if (k0 + q * XS_BLOCK < ne) prod[k0 + q * XS_BLOCK] = p;
+    }
+  }
+}
+
+// f(row, sum of the row's products) for the rows [r0, r1) of a staged block:
+// a wave takes 64 rows at a time, a lane each; the rows longer than
+// XS_CSR_ROW_LANE among them are then summed one by one by the whole wave.
+// Which wave and lane calls f for a row depends on the pattern alone.
+template <class T, class F>
+__device__ __forceinline__ void csr_reduce_rows(const T *prod, int r0, int r1, int e0,
+                                                const int *__restrict__ rp, F &&f) {
+  const int lane = threadIdx.x & (XS_WAVE - 1);
+  for (int b = r0 + (int)(threadIdx.x / XS_WAVE) * XS_WAVE; b < r1; b += XS_BLOCK) {
+    const int r = b + lane;
+    const int a = r < r1 ? rp[r] - e0 : 0, n = r < r1 ? rp[r + 1] - e0 - a : 0;
+    unsigned long long wide = __ballot(n > XS_CSR_ROW_LANE);
+    if (r < r1 && n <= XS_CSR_ROW_LANE) {
+      T s = 0;
+      for (int k = a; k < a + n; ++k) s += prod[k];
+      f(r, s);
+    }
+    while (wide) {   // wave-uniform
+      const int l = __ffsll((long long)wide) - 1;
+      wide &= wide - 1;
+      const int wa = __builtin_amdgcn_readlane(a, l), wn = __builtin_amdgcn_readlane(n, l);
+      double s = 0.0;
+#pragma unroll 4
+      for (int k = lane; k < wn; k += XS_WAVE) s += (double)prod[wa + k];
+      s = wave_sum(s);
+      if (lane == 0) f(b + l, (T)s);
+    }
+  }
+}

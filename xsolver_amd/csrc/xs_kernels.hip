@@ -58,8 +58,9 @@ __device__ __forceinline__ void epilogue_v(int r, double s, double bw, double *_
 
 // ---------------------------------------------------------------------------
 // CSR SpMV: LDS-staged row blocks ("stream" rows of one nnz chunk through LDS
-// with fully coalesced loads of val/colidx, then reduce each row from LDS);
-// rows too long for the LDS tile fall back to one wavefront per row.
+// with fully coalesced loads of val/colidx, then reduce each row from LDS, a
+// lane or a wave per row: csr_reduce_rows); rows too long for the LDS tile
+// fall back to one wavefront per row.
 // Reference kernels replaced: matMultCSR / bmAxCSR
 // (hip/HostMatrix/DeviceMatrix/DeviceMatrixCSR.cpp:59-84, one thread per row).
 // ---------------------------------------------------------------------------
@@ -80,14 +81,10 @@ __global__ __launch_bounds__(XS_BLOCK) void k_spmv_csr(
     const int e0 = rp[r0], e1 = rp[r1];
     const int ne = e1 - e0;
     if (ne <= XS_SPMV_LDS) {
-      for (int k = threadIdx.x; k < ne; k += XS_BLOCK) prod[k] = v[e0 + k] * x[ci[e0 + k]];
+      csr_stage(prod, e0, ne, ci, v, x);
       __syncthreads();
-      for (int r = r0 + threadIdx.x; r < r1; r += XS_BLOCK) {
-        const int a = rp[r] - e0, bnd = rp[r + 1] - e0;
-        double s = 0.0;
-        for (int k = a; k < bnd; ++k) s += prod[k];
-        epilogue<EPI, NV>(r, s, y, b, w, acc);
-      }
+      csr_reduce_rows(prod, r0, r1, e0, rp,
+                      [&](int r, double t) { epilogue<EPI, NV>(r, t, y, b, w, acc); });
     } else {
       const int lane = threadIdx.x & (XS_WAVE - 1);
       for (int r = r0 + (int)(threadIdx.x / XS_WAVE); r < r1; r += XS_BLOCK / XS_WAVE) {

@@ -64,14 +64,10 @@ __global__ __launch_bounds__(XS_BLOCK) void k_spmv_csr32(
     const int e0 = rp[r0], e1 = rp[r1];
     const int ne = e1 - e0;
     if (ne <= XS_SPMV_LDS) {
-      for (int k = threadIdx.x; k < ne; k += XS_BLOCK) prod[k] = v[e0 + k] * x[ci[e0 + k]];
+      csr_stage(prod, e0, ne, ci, v, x);
       __syncthreads();
-      for (int r = r0 + threadIdx.x; r < r1; r += XS_BLOCK) {
-        const int a = rp[r] - e0, bnd = rp[r + 1] - e0;
-        float s = 0.f;
-        for (int k = a; k < bnd; ++k) s += prod[k];
-        epi32<EPI, NV>(r, s, y, b, w, acc);
-      }
+      csr_reduce_rows(prod, r0, r1, e0, rp,
+                      [&](int r, float t) { epi32<EPI, NV>(r, t, y, b, w, acc); });
     } else {
       const int lane = threadIdx.x & (XS_WAVE - 1);
       for (int r = r0 + (int)(threadIdx.x / XS_WAVE); r < r1; r += XS_BLOCK / XS_WAVE) {
