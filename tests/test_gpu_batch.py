@@ -72,3 +72,60 @@ def test_batch_nonzero_x0_uses_initial_residual_base(dev, precision):
                                            x0=x0[lo:hi])
             assert sto == 0 and abs(int(it[s]) - ito) <= 2
             assert np.linalg.norm(x[lo:hi] - xo) / np.linalg.norm(xo) <= X_TOL
+
+
+# rows per system at the edges of k_batch_res: one row, a thread each, 8 rows a
+# thread (its small form), 32 (d in registers), 39 (p in LDS), 50 (its limit),
+# and beyond it (k_batch_cg)
+RES_EDGES = (1, 2, 511, 512, 513, 4095, 4096, 4097, 16384, 16385, 19967, 19968, 19969, 25600,
+             25601)
+
+
+def _band_system(n, kind, rng):
+    """Dominant symmetric systems: 'dia' tridiagonal plus a far pair (5 offsets,
+    diagonal slots), 'wide' with 9 offsets (CSR, rows beyond the 6-entry
+    window), 'unsorted' = tridiagonal with its columns in descending order."""
+    offs = {"dia": (1, 37), "wide": (1, 2, 5, 23), "unsorted": (1,)}[kind]
+    rows, cols, vals = [np.arange(n)], [np.arange(n)], [2.0 * len(offs) + rng.uniform(0.5, 1, n)]
+    for o in offs:
+        if o < n:
+            a = -rng.uniform(0.2, 1, n - o)
+            rows += [np.arange(n - o), np.arange(o, n)]
+            cols += [np.arange(o, n), np.arange(n - o)]
+            vals += [a, a]
+    r, c, v = np.concatenate(rows), np.concatenate(cols), np.concatenate(vals)
+    k = np.lexsort((-c if kind == "unsorted" else c, r))
+    return np.append(0, np.cumsum(np.bincount(r, minlength=n))), c[k], v[k]
+
+
+@pytest.mark.parametrize("precision", [0, 1], ids=["fp64", "fp32"])
+@pytest.mark.parametrize("kind,sizes", [("dia", RES_EDGES), ("wide", RES_EDGES),
+                                        ("unsorted", (1, 513, 4097, 19969)),
+                                        ("dia", (1, 513, 4096)), ("wide", (7, 4095))],
+                         ids=["dia", "wide", "unsorted", "dia-small", "wide-small"])
+def test_batch_resident_edges(dev, kind, sizes, precision):
+    import torch
+    rng = np.random.default_rng(11)
+    sys_ptr, rp, ci, v = batch_concat([_band_system(n, kind, rng) for n in sizes])
+    A = (rp, ci, v)
+    b = gen.spmv(A, rng.uniform(-1, 1, int(sys_ptr[-1])))
+    say(f"[batch edges] {kind} rows={sys_ptr[-1]} precision={precision}")
+    B = XBatch(sys_ptr, *A)
+    x, st = B.solve(b, tol=1e-9, maxiter=500, precision=precision)
+    it, rr = B.results()
+    B.close()
+    assert st == 0 and rr.max() < 1e-9
+    xo, ito, _, bad = oracle.batch_cg(sys_ptr, A, b, tol=1e-9, maxiter=500)
+    assert bad == 0
+    for s, (lo, hi) in enumerate(zip(sys_ptr[:-1], sys_ptr[1:])):
+        dx = np.linalg.norm(x[lo:hi] - xo[lo:hi]) / np.linalg.norm(xo[lo:hi])
+        # FP64: the oracle's recurrence; FP32: both meet the residual
+        # tolerance, and the matrices' condition is below 20
+        assert dx <= (X_TOL if precision == 0 else 2 * 20 * 1e-9), (hi - lo, dx)
+        if precision == 0:
+            assert abs(int(it[s]) - int(ito[s])) <= 1, (hi - lo, it[s], ito[s])
+    if precision == 0:   # the allocation-free entry: the same systems, bit for bit
+        from tests.test_zz_no_alloc import _noalloc
+        rc, x2, it2, rr2, _ = _noalloc(torch, dev, sys_ptr, rp, ci, v, b, 1e-9, 500)
+        assert rc == 0 and np.array_equal(x2, x) and np.array_equal(it2, it)
+        assert np.array_equal(rr2, rr)

@@ -9,6 +9,7 @@
 
 #include "../../include/xsolver_c.h"
 #include "xs_batch.h"
+#include "xs_internal.h"
 
 struct xs_batch {
   hipStream_t stream = nullptr;
@@ -18,6 +19,13 @@ struct xs_batch {
   double *v = nullptr, *dinv = nullptr, *w64 = nullptr, *b = nullptr, *x = nullptr;
   double *relres = nullptr;
   float *v32 = nullptr, *dinv32 = nullptr, *w32 = nullptr;
+  // systems by size, largest first: nbig of more than BT_RES_ROWS rows
+  // (k_batch_cg), then those that k_batch_res takes, of at most resrows rows
+  int nbig = 0, resrows = 0;
+  // diagonal slots of every system (when each has few), read by k_batch_res
+  int *off = nullptr;
+  double *dv = nullptr;
+  float *dv32 = nullptr;
   unsigned *queue = nullptr;
   int *iters = nullptr, *bad = nullptr;
   float ms = 0.f;
@@ -46,7 +54,7 @@ extern "C" int xs_batch_destroy(xs_batch *bt) {
   auto f = [](auto *&p) { if (p) (void)hipFree((void *)p); p = nullptr; };
   f(bt->sys_ptr); f(bt->order); f(bt->rp); f(bt->ci); f(bt->v); f(bt->dinv); f(bt->w64);
   f(bt->b); f(bt->x); f(bt->relres); f(bt->v32); f(bt->dinv32); f(bt->w32); f(bt->queue);
-  f(bt->iters); f(bt->bad);
+  f(bt->iters); f(bt->bad); f(bt->off); f(bt->dv); f(bt->dv32);
   if (bt->e0) (void)hipEventDestroy(bt->e0);
   if (bt->e1) (void)hipEventDestroy(bt->e1);
   if (bt->stream) (void)hipStreamDestroy(bt->stream);
@@ -84,14 +92,19 @@ extern "C" int xs_batch_create(xs_batch **out, int nsys, const int *sys_ptr, con
   std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
     return sys_ptr[a + 1] - sys_ptr[a] > sys_ptr[b + 1] - sys_ptr[b];
   });
+  auto rows = [&](int q) { return sys_ptr[order[q] + 1] - sys_ptr[order[q]]; };
+  while (bt->nbig < nsys && rows(bt->nbig) > BT_RES_ROWS) ++bt->nbig;
+  bt->resrows = bt->nbig < nsys ? rows(bt->nbig) : 0;
+  // k_batch_cg keeps six vectors in the workspace, k_batch_res at most p and d
+  const size_t wvecs = bt->nbig ? 6 : 2;
   if ((rc = bt_alloc(&bt->sys_ptr, nsys + 1)) || (rc = bt_alloc(&bt->order, nsys)) ||
       (rc = bt_alloc(&bt->rp, n + 1)) || (rc = bt_alloc(&bt->ci, nnz)) ||
       (rc = bt_alloc(&bt->v, nnz)) || (rc = bt_alloc(&bt->dinv, n)) ||
-      (rc = bt_alloc(&bt->w64, 6 * (size_t)n)) || (rc = bt_alloc(&bt->b, n)) ||
+      (rc = bt_alloc(&bt->w64, wvecs * n)) || (rc = bt_alloc(&bt->b, n)) ||
       (rc = bt_alloc(&bt->x, n)) || (rc = bt_alloc(&bt->relres, nsys)) ||
-      (rc = bt_alloc(&bt->v32, nnz)) || (rc = bt_alloc(&bt->dinv32, n)) ||
-      (rc = bt_alloc(&bt->w32, 6 * (size_t)n)) || (rc = bt_alloc(&bt->queue, 4)) ||
-      (rc = bt_alloc(&bt->iters, nsys)) || (rc = bt_alloc(&bt->bad, 1))) {
+      (rc = bt_alloc(&bt->dinv32, n)) || (rc = bt_alloc(&bt->off, (size_t)nsys * XS_DIA_MAX)) ||
+      (rc = bt_alloc(&bt->w32, wvecs * n)) || (rc = bt_alloc(&bt->queue, 4)) ||
+      (rc = bt_alloc(&bt->iters, nsys)) || (rc = bt_alloc(&bt->bad, 4))) {
     xs_batch_destroy(bt);
     return rc;
   }
@@ -100,6 +113,26 @@ extern "C" int xs_batch_create(xs_batch **out, int nsys, const int *sys_ptr, con
   BT_CHK(hipMemcpy(bt->rp, rowptr, sizeof(int) * (n + 1), hipMemcpyHostToDevice));
   BT_CHK(hipMemcpy(bt->ci, colidx, sizeof(int) * nnz, hipMemcpyHostToDevice));
   BT_CHK(hipMemcpy(bt->v, val, sizeof(double) * nnz, hipMemcpyHostToDevice));
+  // the systems' diagonal offsets, and slots when every system has few
+  int stat[2] = {0, 0};
+  BT_CHK(hipMemset(bt->bad, 0, 2 * sizeof(int)));
+  xs_batch_offsets(bt->stream, nsys, bt->sys_ptr, bt->rp, bt->ci, bt->off, bt->bad);
+  BT_CHK(hipMemcpyAsync(stat, bt->bad, sizeof(stat), hipMemcpyDeviceToHost, bt->stream));
+  BT_CHK(hipStreamSynchronize(bt->stream));
+  if (!stat[1] && stat[0] <= BT_RES_ND && bt->resrows) {
+    if ((rc = bt_alloc(&bt->dv, (size_t)BT_RES_ND * n)) ||
+        (rc = bt_alloc(&bt->dv32, (size_t)BT_RES_ND * n))) {
+      xs_batch_destroy(bt);
+      return rc;
+    }
+    xs_batch_dia(bt->stream, nsys, n, bt->sys_ptr, bt->off, bt->rp, bt->ci, bt->v, bt->dv,
+                 bt->dv32);
+  }
+  // the CSR values in FP32: only where a kernel reads them
+  if ((!bt->dv || bt->nbig) && (rc = bt_alloc(&bt->v32, nnz))) {
+    xs_batch_destroy(bt);
+    return rc;
+  }
   BT_CHK(hipMemset(bt->bad, 0x7f, sizeof(int)));
   xs_batch_prep(bt->stream, n, bt->rp, bt->ci, bt->v, bt->dinv, bt->dinv32, bt->v32, bt->bad);
   int bad = 0;
@@ -120,12 +153,23 @@ static int batch_run(xs_batch *bt, const double *d_b, double *d_x, double tol, i
   int dev = 0, cus = 256;
   (void)hipGetDevice(&dev);
   (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-  const int grid = std::min(bt->nsys, 2 * cus);
-  BT_CHK(hipMemsetAsync(bt->queue, 0, sizeof(unsigned), s));
+  BT_CHK(hipMemsetAsync(bt->queue, 0, 2 * sizeof(unsigned), s));
   BT_CHK(hipEventRecord(bt->e0, s));
-  xs_batch_cg(s, grid, bt->nsys, bt->n, bt->nnz, bt->order, bt->sys_ptr, bt->rp, bt->ci, bt->v, bt->v32,
-              bt->dinv, bt->dinv32, d_b, d_x, bt->w64, bt->w32, tol, maxiter, precision, 1e-2,
-              bt->queue, bt->iters, bt->relres);
+  xs_batch_args P;
+  P.N = bt->n; P.nnz = bt->nnz;
+  P.order = bt->order; P.sys_ptr = bt->sys_ptr; P.rp = bt->rp; P.ci = bt->ci;
+  P.v = bt->v; P.v32 = bt->v32;
+  P.off = bt->off; P.dv = bt->dv; P.dv32 = bt->dv32;
+  P.dinv = bt->dinv; P.dinv32 = bt->dinv32;
+  P.b = d_b; P.x = d_x; P.w64 = bt->w64; P.w32 = bt->w32;
+  P.tol = tol; P.inner_tol = 1e-2; P.maxiter = maxiter;
+  P.queue = bt->queue; P.iters = bt->iters; P.relres = bt->relres;
+  xs_batch_cg(s, std::min(bt->nbig, 2 * cus), bt->nbig, BT_RES_ROWS, precision, P);
+  P.order = bt->order + bt->nbig;
+  P.queue = bt->queue + 1;
+  const int nres = bt->nsys - bt->nbig;
+  if (!xs_batch_res(s, std::min(nres, 2 * cus), nres, bt->resrows, precision, P))
+    return XS_ERR_DEVICE;
   BT_CHK(hipGetLastError());
   BT_CHK(hipEventRecord(bt->e1, s));
   BT_CHK(hipEventSynchronize(bt->e1));
@@ -172,13 +216,13 @@ extern "C" double xs_batch_get_time_ms(const xs_batch *bt) { return bt ? bt->ms 
 // ---------------------------------------------------------------------------
 // Allocation-free batched solve (no reference counterpart).  For callers that
 // cannot allocate device memory (code under HIP graph capture, serving loops,
-// harnesses that forbid hipMalloc).  Its workspace -- the work-queue counter,
+// harnesses that forbid hipMalloc).  Its workspace -- the work-queue counters,
 // 1/a_ii and the six CG vectors, 7 doubles per row -- lives in `scratch`, a
 // static device array of fixed size that each GPU holds until the process
 // ends.  Calls on one GPU share that GPU's array (the last call's contents
 // stay in it): calls that overlap on one GPU, on any streams, race.
 // ---------------------------------------------------------------------------
-#define XS_NOALLOC_HEADER 256   // bytes before the vectors: the queue counter
+#define XS_NOALLOC_HEADER 256   // bytes before the vectors: the queue counters
 static __device__ __align__(256) unsigned char
     scratch[XS_NOALLOC_HEADER + 7 * sizeof(double) * (size_t)XS_BATCH_NOALLOC_MAX_ROWS];
 
@@ -224,12 +268,19 @@ extern "C" int xs_batch_solve_noalloc(int nsys, int n, int nnz, const int *d_sys
   (void)hipGetDevice(&dev);
   (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
   const int grid = std::min(nsys, 2 * cus);
-  // one launch sets 1/a_ii and clears the queue counter (kernels only, so the
-  // call can be captured into a graph)
+  // one launch sets 1/a_ii and clears the queue counters (kernels only, so the
+  // call can be captured into a graph); the sizes of the systems are on the
+  // device, so each of the two kernels passes over the other's
   xs_batch_prep64(s, n, d_rowptr, d_colidx, d_val, dinv, queue);
-  xs_batch_cg(s, grid, nsys, n, nnz, nullptr, d_sys_ptr, d_rowptr, d_colidx, d_val, nullptr,
-              dinv, nullptr, d_rhs, d_sol, w64, nullptr, tol, maxiter, 0, 0.0, queue, d_iters,
-              d_relres);
+  xs_batch_args P;
+  P.N = n; P.nnz = nnz;
+  P.sys_ptr = d_sys_ptr; P.rp = d_rowptr; P.ci = d_colidx; P.v = d_val;
+  P.dinv = dinv; P.b = d_rhs; P.x = d_sol; P.w64 = w64;
+  P.tol = tol; P.maxiter = maxiter;
+  P.queue = queue; P.iters = d_iters; P.relres = d_relres;
+  if (n > BT_RES_ROWS) xs_batch_cg(s, grid, nsys, BT_RES_ROWS, 0, P);
+  P.queue = queue + 1;
+  if (!xs_batch_res(s, grid, nsys, std::min(n, BT_RES_ROWS), 0, P)) return XS_ERR_DEVICE;
   if (hipGetLastError() != hipSuccess) return XS_ERR_DEVICE;
   return XS_OK;
 }

@@ -2,6 +2,8 @@
 // wave / workgroup sums and the "last workgroup" grid reduction that runs the
 // Krylov scalar updates (do_finish) on the device.
 #pragma once
+#include <climits>
+
 #include "xs_internal.h"
 
 // ---------------------------------------------------------------------------
@@ -408,4 +410,16 @@ __device__ __forceinline__ void csr_reduce_rows(const T *prod, int r0, int r1, i
       if (lane == 0) f(b + l, (T)s);
     }
   }
+}
+
+// Offset o into a table of XS_DIA_MAX slots (INT_MIN: free); false when it is
+// full of others.  A slot only ever changes from INT_MIN to its offset, so a
+// plain read that finds the offset is final and a CAS claims a free slot.
+__device__ __forceinline__ bool dia_insert(int *tab, int o) {
+  for (int k = 0; k < XS_DIA_MAX; ++k) {
+    int cur = tab[k];
+    if (cur == INT_MIN) cur = atomicCAS(tab + k, INT_MIN, o);
+    if (cur == INT_MIN || cur == o) return true;
+  }
+  return false;
 }

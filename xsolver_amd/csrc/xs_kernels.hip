@@ -526,20 +526,10 @@ void xs_build_ell(hipStream_t s, const xs_csr &A, int W, xs_ell &E) {
 
 // Distinct offsets column - row, gathered into t[0 .. XS_DIA_MAX) (INT_MIN:
 // free slot); t[XS_DIA_MAX] = 1 when there are more, or a row repeats a
-// column.  A slot only ever changes from INT_MIN to its offset, so a plain
-// read that finds the offset is final and a CAS claims a free slot.  Each
+// column (dia_insert in xs_device.h).  Each
 // workgroup collects into an LDS table first and merges its (at most
 // XS_DIA_MAX) offsets into t at the end: the global table sees a handful of
 // atomics per workgroup instead of a read per entry.
-__device__ __forceinline__ bool dia_insert(int *tab, int o) {
-  for (int k = 0; k < XS_DIA_MAX; ++k) {
-    int cur = tab[k];
-    if (cur == INT_MIN) cur = atomicCAS(tab + k, INT_MIN, o);
-    if (cur == INT_MIN || cur == o) return true;
-  }
-  return false;
-}
-
 // part: 0 all entries, 1 strictly lower, 2 strictly upper (dpos: pivots)
 __global__ __launch_bounds__(256) void k_dia_offsets(int n, const int *__restrict__ rp,
                                                      const int *__restrict__ ci,
