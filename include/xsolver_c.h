@@ -123,7 +123,8 @@ int xs_pc_setilut(xs_ctx *ctx, double tol, int max_fill);
  *                    (default) = a separate update kernel
  *   "use_graph"      1 = replay each batch of check_every iterations as a
  *                    captured HIP graph, 0 = launch kernels one by one,
- *                    -1 (default) = graphs for k-RHS block solves only (a
+ *                    -1 (default) = graphs for k-RHS block solves only, and CG
+ *                    in one launch where cg_resident allows it (a
  *                    single solve's short kernels ran faster launched one by
  *                    one, and its graph is captured anew in every solve)
  *   "precision"      0 = FP64, 1 = FP32 inner Krylov solve inside FP64
@@ -180,6 +181,10 @@ int xs_pc_setilut(xs_ctx *ctx, double tol, int max_fill);
  *                    1 = row-binned vector CSR (lanes per row = mean row length
  *                    rounded up to a power of two, long rows one wavefront
  *                    each).  0 and 1 also drop the automatic ELL copy.
+ *   "cg_resident"    1 (default) = CG with Jacobi or no preconditioner runs as
+ *                    one launch when A has a diagonal-slot copy (spmv_dia) and
+ *                    its rows and reach fit the chip; 0 = a launch per kernel.
+ *                    Not used with use_graph = 0 or 1 or while "profile" is on
  *   "use_ell"        1 = ELL SpMV (same as advanced_pam[1] = 1)
  *   "spmv_dia"       1 (default) = when the ELL copy is built and the matrix
  *                    has at most 8 distinct column - row offsets (5- and

@@ -616,3 +616,81 @@ def test_matrix_market_input_solve(dev, tmp_path):
     g2 = gpu_solve((rp2, ci2, v2), b, "bicgstab", "ilu0", 1e-10, 300, parilu_async=0)
     assert np.array_equal(g1["x"], g2["x"]) and g1["it"] == g2["it"]
     g1["S"].close(); g2["S"].close()
+
+
+def _tridiag(n):
+    i = np.arange(n)
+    r = np.concatenate([i, i[1:], i[:-1]])
+    c = np.concatenate([i, i[:-1], i[1:]])
+    v = np.concatenate([np.full(n, 2.5), np.full(2 * n - 2, -1.0)])
+    k = np.lexsort((c, r))
+    return (np.append(0, np.cumsum(np.bincount(r, minlength=n))).astype(np.int32),
+            c[k].astype(np.int32), v[k])
+
+
+def _grid2d(nx, ny):
+    return gen.vardiff2d(np.exp(0.3 * np.random.default_rng(nx + ny).standard_normal((ny, nx))))
+
+
+# rows at the edges of the one-launch CG: one row, one workgroup with 2 / 4 / 8
+# rows a thread, the first sizes of several workgroups, a last workgroup with
+# one row, a reach beyond a workgroup's rows, and 7 slots
+CG_RES = {"tri1": lambda: _tridiag(1), "tri512": lambda: _tridiag(512),
+          "tri1024": lambda: _tridiag(1024), "tri1025": lambda: _tridiag(1025),
+          "tri2049": lambda: _tridiag(2049), "tri4096": lambda: _tridiag(4096),
+          "tri4097": lambda: _tridiag(4097), "tri8193": lambda: _tridiag(8193),
+          "tri16385": lambda: _tridiag(16385), "tri36865": lambda: _tridiag(36865),
+          "grid47x61": lambda: _grid2d(47, 61), "grid2000x3": lambda: _grid2d(2000, 3),
+          "grid3x2000": lambda: _grid2d(3, 2000), "grid5000x9": lambda: _grid2d(5000, 9),
+          "grid191x193": lambda: _grid2d(191, 193), "poisson3d_12": lambda: gen.convdiff3d(12, pe=0.0),
+          "poisson3d_37": lambda: gen.convdiff3d(37, pe=0.0)}
+
+
+@pytest.mark.parametrize("pc", ["jacobi", "none"])
+@pytest.mark.parametrize("name", list(CG_RES))
+def test_cg_one_launch_matches_kernel_loop(dev, name, pc):
+    """CG in one launch against the loop of kernels: the same recurrence with
+    the partial sums of the inner products in another order, so the same
+    iteration count, and residuals and solutions to rounding times the
+    iterations it has grown over."""
+    A = CG_RES[name]()
+    n = len(A[0]) - 1
+    rng = np.random.default_rng(6)
+    b, x0 = gen.spmv(A, rng.uniform(-1, 1, n)), rng.uniform(-1, 1, n)
+    say(f"[cg one launch] {name} n={n} {pc}")
+    out = []
+    for resident in (0, 1):
+        S = XSolver()
+        S.mat_setup(*A)
+        S.ksp_settype("cg")
+        S.ksp_setoption(1e-9, 2000)
+        S.pc_settype(pc)
+        S.set_option("use_ell", 1)
+        S.set_option("cg_resident", resident)
+        assert S.time_ms("spmv:dia") > 0
+        x, st = S.solve(b, x0=x0)
+        runs = [(x, st, S.iterations, S.residual, S.initial_residual, S.resvec())]
+        x, st = S.solve(np.zeros(n))                    # a zero residual
+        runs.append((x, st, S.iterations, S.residual, S.initial_residual, S.resvec()))
+        S.ksp_set_absolute_tol(1e30)                    # converged at once
+        x, st = S.solve(b, x0=x0)
+        runs.append((x, st, S.iterations, S.residual, S.initial_residual, S.resvec()))
+        S.ksp_set_absolute_tol(0.0)
+        S.ksp_setoption(1e-30, 3)                       # out of iterations
+        x, st = S.solve(b)
+        runs.append((x, st, S.iterations, S.residual, S.initial_residual, S.resvec()))
+        S.close()
+        out.append(runs)
+    eps = 2.3e-16
+    for (x0_, st0, it0, rl0, r00, rv0), (x1, st1, it1, rl1, r01, rv1) in zip(*out):
+        assert st0 == st1 and it0 == it1 and len(rv0) == len(rv1), (st0, st1, it0, it1)
+        tol = 64 * eps * (it0 + 1)
+        assert np.linalg.norm(x0_ - x1) <= 100 * tol * max(np.linalg.norm(x0_), 1e-300)
+        assert abs(r00 - r01) <= tol * r00
+        # a difference of eps in an inner product grows with the loss of
+        # orthogonality, which follows the convergence of the extreme Ritz
+        # values: over the first 20 iterations of these systems (condition up
+        # to 1e4) by less than 1e6, the bound of the oracle comparisons; later
+        # residuals agree in size only
+        assert np.all(np.abs(rv0 - rv1)[:20] <= 1e-6 * rv0[:20] + 4 * eps * r00)
+        assert np.all(rv1 <= 2 * rv0 + 4 * eps * r00)

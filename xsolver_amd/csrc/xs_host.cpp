@@ -832,6 +832,7 @@ extern "C" int xs_set_option(xs_ctx *c, const char *name, double value) {
     c->trsv_wg = (int)value;
     c->ilu.trsv_wg = c->trsv_wg;
   }
+  else if (k == "cg_resident") { c->cg_resident = value != 0; }
   else if (k == "spmv_dia") {   // 1: diagonal-slot copy for the FP64 SpMV when possible
     if (value < 0 || value > 1) return XS_ERR_ARG;
     c->spmv_dia = value != 0;

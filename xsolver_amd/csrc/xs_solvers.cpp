@@ -7,8 +7,10 @@
 
 #include <algorithm>
 #include <cstdio>
+#include <cstdlib>
 
 #include "../../include/xsolver_c.h"
+#include "xs_cgres.h"
 #include "xs_intel.h"
 #include "xs_krylov.h"
 #include "xs_mixed.h"
@@ -18,6 +20,17 @@
   do {                                          \
     if ((call) != hipSuccess) return XS_ERR_DEVICE; \
   } while (0)
+
+// status of a solve whose state is in the pinned mirror
+static int solve_status(xs_ctx *c) {
+  const xs_state &h = *c->h_state;
+  c->iters = h.iter;
+  c->res0 = h.sc[S_RES0];
+  c->resl = h.sc[S_RESL];
+  if (h.done == 2) return XS_ERR_BREAKDOWN;
+  if (h.done == 1) return XS_OK;
+  return XS_NOT_CONVERGED;
+}
 
 // Launch `iteration` until the device reports convergence/breakdown or
 // maxiter iterations have been launched.  Two pinned state slots are used so
@@ -37,18 +50,60 @@ static int drive(xs_ctx *c, F iteration) {
     XS_CHK(hipMemcpyAsync(c->h_state, c->st, sizeof(xs_state), hipMemcpyDeviceToHost, s));
     XS_CHK(hipStreamSynchronize(s));
   }
-  const xs_state &h = *c->h_state;
-  c->iters = h.iter;
-  c->res0 = h.sc[S_RES0];
-  c->resl = h.sc[S_RESL];
-  if (h.done == 2) return XS_ERR_BREAKDOWN;
-  if (h.done == 1) return XS_OK;
-  return XS_NOT_CONVERGED;
+  return solve_status(c);
+}
+
+// CG with Jacobi or no preconditioner in one launch (xs_cgres.hip) when A has
+// a diagonal-slot copy and its rows and reach fit; *used = 0: not launched.
+// Not while kernels are timed one by one, nor when use_graph says how the
+// kernels of an iteration are launched.
+static int cg_resident(xs_ctx *c, const double *b, double *x, int *used) {
+  *used = 0;
+  if (!c->cg_resident || c->use_t || c->prof_kind != 0 || c->use_graph >= 0 ||
+      !(c->pc == XS_PC_JACOBI || c->pc == XS_PC_NONE) || !(c->use_ell && c->ell.dv))
+    return XS_OK;
+  xs_cgres_args A;
+  A.n = c->A.n;
+  A.ld = c->ell.ld;
+  A.nd = c->ell.nd;
+  A.off = c->ell.doff;
+  for (int k = 0; k < A.nd; ++k) A.reach = std::max(A.reach, std::abs(A.off.o[k]));
+  const size_t words = xs_cgres_words(A.n, A.reach);
+  if (!words) return XS_OK;
+  if (c->cg_words < words) {
+    if (c->cg_buf) (void)hipFree(c->cg_buf);
+    c->cg_buf = nullptr;
+    c->cg_words = 0;
+    if (hipMalloc((void **)&c->cg_buf, sizeof(unsigned long long) * words) != hipSuccess) {
+      (void)hipGetLastError();
+      return XS_OK;   // the loop of kernels needs no such buffer
+    }
+    c->cg_words = words;
+  }
+  A.dv = c->ell.dv;
+  A.dinv = c->pc == XS_PC_JACOBI ? c->jac_dinv : nullptr;
+  A.b = b;
+  A.x = x;
+  A.tol = c->tol;
+  A.abstol = c->abstol;
+  A.maxiter = c->maxiter;
+  A.st = c->st;
+  A.resvec = c->resvec_d;
+  A.err = c->counters;
+  A.slots = c->cg_buf;
+  A.z = c->cg_buf + 8 * CR_MAX_WG;
+  if (!xs_cgres(c->stream, A)) return XS_OK;
+  *used = 1;
+  XS_CHK(hipMemcpyAsync(c->h_state, c->st, sizeof(xs_state), hipMemcpyDeviceToHost, c->stream));
+  XS_CHK(hipStreamSynchronize(c->stream));
+  return solve_status(c);
 }
 
 // Preconditioned CG, hip/Solver/xsolver_cg.cpp:16-74.
 int xs_solve_cg(xs_ctx *c, const double *b, double *x) {
-  int rc = xs_ctx_ensure_work(c, XS_NWORK);
+  int used = 0, rc = cg_resident(c, b, x, &used);
+  if (used) return rc;
+  rc = xs_ctx_ensure_work(c, XS_NWORK);
   if (rc) return rc;
   const int n = c->A.n;
   hipStream_t s = c->stream;
@@ -493,6 +548,9 @@ int xs_solve_ibicgstab(xs_ctx *c, const double *b, double *x) {
 
 void xs_solvers_free(xs_ctx *c) {
   xs_multi_free(c);
+  if (c->cg_buf) (void)hipFree(c->cg_buf);
+  c->cg_buf = nullptr;
+  c->cg_words = 0;
   if (c->mdot_partial) (void)hipFree(c->mdot_partial);
   c->mdot_partial = nullptr;
   c->mdot_len = 0;

@@ -55,6 +55,7 @@ struct xs_ctx {
   int trsv_wg = 256;            // persistent workgroups of the SpTRSV
   int trsv_prog = -1;           // SpTRSV group mode (xs_tsched::prog), -1 = by factor width
   int trsv_gather = 0;          // SpTRSV gather width (4 or 16), 0 = by factor width
+  bool cg_resident = true;      // CG + Jacobi / none in one launch when the system allows it
   bool spmv_dia = true;         // diagonal-slot copy of A for the FP64 SpMV when possible
   bool sweep_dia = true;        // diagonal-slot copies of L / U for the FP64 sweeps
   bool parilu_dia = true;       // ParILU(0) sweeps over diagonal slots when possible
@@ -102,6 +103,8 @@ struct xs_ctx {
   double *small_d = nullptr;
   size_t small_len = 0;
   double *ts_partial = nullptr;
+  unsigned long long *cg_buf = nullptr;   // exchange words of the one-launch CG
+  size_t cg_words = 0;
   double *mdot_partial = nullptr;   // intel-family multi-dot partials
   size_t mdot_len = 0;
   size_t ts_partial_len = 0;
