@@ -162,6 +162,11 @@ int xs_pc_setilut(xs_ctx *ctx, double tol, int max_fill);
  *                    ILUT, precon_gpuilut.cpp:19-20)
  *   "trsv_schedule"  1 (default) = hand out the triangular-solve row groups in
  *                    dependency-level order, 0 = row order
+ *   "trsv_chains"    1 (default) = FP64 triangular solves of one right-hand
+ *                    side with narrow factors (ILU(0) of 5- and 7-point grids)
+ *                    run over chains of row groups, a wave per chain, where the
+ *                    pattern has them (xs_get_time_ms("trsv:chains") tells);
+ *                    0 or trsv_progressive = 1 = the general solve
  *   "trsv_progressive" -1 (default) = by factor width: factors with more than
  *                    six entries per row and triangle solve every 64-row group
  *                    lane by lane, publishing each row as soon as it is final;

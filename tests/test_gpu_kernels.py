@@ -542,3 +542,80 @@ def test_csr_row_blocks_mixed_lengths(dev, lens):
         xs, st = S.solve(b)
         assert st == 0 and true_relres(A, b, xs) < 1e-10
     S.close()
+
+
+def _grid_stencil(dims, offs, seed):
+    """Random nonsymmetric stencil matrix on a grid, entries in [-1, 1], the
+    diagonal 2.2 times their number."""
+    cols, mask = gen._grid_offsets(dims, offs)
+    n = len(cols)
+    rng = np.random.default_rng(seed)
+    v = np.where(mask, rng.uniform(-1, 1, cols.shape), 0.0)
+    d = offs.index((0,) * len(dims))
+    v[:, d] = 2.2 * (len(offs) - 1)
+    return gen._assemble(n, cols, v, mask)
+
+
+S5 = [(0, -1), (-1, 0), (0, 0), (1, 0), (0, 1)]
+S7 = [(0, 0, -1), (0, -1, 0), (-1, 0, 0), (0, 0, 0), (1, 0, 0), (0, 1, 0), (0, 0, 1)]
+S9 = [(0, 0, -1), (0, -2, 0)] + S7[1:6] + [(0, 2, 0), (0, 0, 1)]
+S9D = [(0, 0, -1), (1, 0, -1)] + S7[1:6] + [(-1, 0, 1), (0, 0, 1)]
+CHAINS = {  # grid, stencil, chains of L (0: the general solve)
+    "one_narrow": ((17, 40), S5, 1),          # part of a wave
+    "one_full": ((64, 9), S5, 1),             # a step past a block of 8
+    "carry_one_lane": ((65, 30), S5, 2),      # a group of one lane, carried
+    "four": ((256, 300), S5, 4),              # chain 0 has less to do: the pace
+    "next_workgroup": ((300, 100), S5, 5),
+    "eight_waves": ((520, 30), S5, 9),        # more chains per step: 8 to a workgroup
+    "planes": ((20, 20, 24), S7, 20),
+    "planes_carry": ((70, 12, 10), S7, 24),
+    "three_entries": ((128, 9, 16), S9, 18),  # and a carry
+    "own_ring": ((60, 9, 16), S9D, 9),        # another lane of the chain's last step
+    "groups_too_short": ((12, 12, 12), S7, 0),
+    "chains_too_short": ((40, 40, 5), S7, 0),
+}
+
+
+@pytest.mark.parametrize("name", list(CHAINS))
+def test_trsv_chains_edges(dev, name):
+    """The triangular solves over chains against the oracle and, transposed,
+    against the general solve.  The off-diagonal factor entries of every row
+    and column sum to q < 0.5 of the pivot, so the error of x is at most
+    1 / (1 - q) = 2 times a row's own, which a scan of 64 affine maps (two
+    roundings each) and four products bound by 140 eps: 2 * 140 * 2.2e-16 =
+    6.2e-14 of max |x|.  Over both triangles of two solves that differ by as
+    much each: 2 * (6.2e-14 + 2 * 6.2e-14)."""
+    import torch
+    dims, offs, chains = CHAINS[name]
+    A = _grid_stencil(dims, offs, 11)
+    n = len(A[0]) - 1
+    say(f"[chains] {name} n={n}")
+    b = np.random.default_rng(6).uniform(-1, 1, n)
+    bd = dev_tensor(b, dev)
+    out = {}
+    for on in (1, 0):
+        S = XSolver()
+        S.mat_setup(*A)
+        S.pc_settype("ilu0")
+        S.set_option("parilu_async", 0)
+        S.set_option("trsv_chains", on)
+        S.pc_setup()
+        ld, ud, td = (torch.empty(n, dtype=torch.float64, device=dev) for _ in range(3))
+        for rep in range(2):   # tickets reset themselves
+            S.trsv(0, bd, ld, torch_stream())
+            S.trsv(1, bd, ud, torch_stream())
+            S.pc_apply_t(bd, td, torch_stream())
+            torch.cuda.synchronize()
+        assert S.time_ms("trsv:chains") == (chains if on else -1)   # -1: not looked at
+        out[on] = [t.cpu().numpy() for t in (ld, ud, td)]
+        if on:
+            L, U, dinv = split_factors(*S.factors(n, len(A[2])))
+        S.close()
+    rl, ru = (np.repeat(np.arange(n), np.diff(T[0])) for T in (L, U))
+    ad = np.abs(dinv)
+    for idx, w in ((rl, np.abs(L[2])), (L[1], np.abs(L[2])), (ru, np.abs(U[2]) * ad[ru]),
+                   (U[1], np.abs(U[2]) * ad[U[1]])):
+        assert np.bincount(idx, w, n).max() < 0.5
+    assert rel_err(out[1][0], oracle.lower_solve(L, b)) < 6.2e-14
+    assert rel_err(out[1][1], oracle.upper_solve(U, dinv, b)) < 6.2e-14
+    assert rel_err(out[1][2], out[0][2]) < 6 * 6.2e-14

@@ -66,6 +66,15 @@ __device__ __forceinline__ double dpp_d(double v, double ident) {
   return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) |
                                           (unsigned long long)(unsigned)lo));
 }
+// identity 0 for every lane without a source: by the instruction itself
+template <int CTRL>
+__device__ __forceinline__ double dpp_d0(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)(b & 0xffffffff), CTRL, 0xF, 0xF, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xF, 0xF, true);
+  return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) |
+                                          (unsigned long long)(unsigned)lo));
+}
 template <int CTRL, int ROWMASK>
 __device__ __forceinline__ float dpp_f(float v, float ident) {
   return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(ident), __float_as_int(v), CTRL,
@@ -75,7 +84,8 @@ template <int CTRL, int ROWMASK, int KC>
 __device__ __forceinline__ void affine_step(double (&c)[KC], double &m) {
   const double mj = dpp_d<CTRL, ROWMASK>(m, 1.0);
 #pragma unroll
-  for (int q = 0; q < KC; ++q) c[q] = c[q] + m * dpp_d<CTRL, ROWMASK>(c[q], 0.0);
+  for (int q = 0; q < KC; ++q)
+    c[q] = c[q] + m * (ROWMASK == 0xF ? dpp_d0<CTRL>(c[q]) : dpp_d<CTRL, ROWMASK>(c[q], 0.0));
   m = m * mj;
 }
 template <int CTRL, int ROWMASK>

@@ -77,8 +77,10 @@ static void free_precond(xs_ctx *c) {
   dfree(F.tl.ci); dfree(F.tl.v); dfree(F.tl.vlo); dfree(F.tl.co); dfree(F.tl.ww);
   dfree(F.tu.ci); dfree(F.tu.v); dfree(F.tu.vlo); dfree(F.tu.co); dfree(F.tu.ww); dfree(F.tu.vs);
   dfree(F.tl.dv); dfree(F.tu.dv); dfree(F.tu.dvs); dfree(F.tl.dvlo); dfree(F.tu.dvlo);
+  for (xs_strip *S : {&F.sl, &F.su, &F.tsl, &F.tsu}) xs_strip_free(*S);
   c->tell_ready = c->tell32_ready = false;
   F = xs_ilu();
+  F.chains = c->trsv_chains;
   F.trsv_wg = c->trsv_wg;
   F.trsv_prog = c->trsv_prog;
   F.trsv_gather = c->trsv_gather;
@@ -438,14 +440,15 @@ static std::string shape_key(const char *kind, const int *hrp, int n, int nnz) {
   return buf;
 }
 
-static int ensure_trsv_sched(xs_ctx *c, bool exact = false);
+enum { NEED_CHAINS = 1, NEED_GROUPS = 2 };   // forms of the exact triangular solves
+static int ensure_trsv_sched(xs_ctx *c, bool exact, int need);
 
 // The triangular solves of a set-up factor: persistent workgroups, gather
 // width and group mode, each combination timed on a lower plus an upper
 // solve; the fastest is kept (and cached by the factor's shape).
 static int tune_trsv(xs_ctx *c) {
   int rc;
-  if ((rc = ensure_trsv_sched(c, true))) return rc;
+  if ((rc = ensure_trsv_sched(c, true, NEED_CHAINS | NEED_GROUPS))) return rc;
   xs_ilu &F = c->ilu;
   std::vector<int> hrp(F.n + 1);
   XS_HIP(hipStreamSynchronize(c->stream));
@@ -849,10 +852,16 @@ extern "C" int xs_set_option(xs_ctx *c, const char *name, double value) {
     if (value < 0 || value > 1) return XS_ERR_ARG;
     if ((value != 0) != c->parilu_dia) { c->parilu_dia = value != 0; free_precond(c); }
   }
+  else if (k == "trsv_chains") {   // 1: FP64 solves of narrow factors over chains of groups
+    c->trsv_chains = value != 0;
+    c->ilu.chains = c->trsv_chains;
+    c->ilu.have_t = false;
+  }
   else if (k == "trsv_progressive") {   // -1 auto, 0 scan chain groups, 1 lane by lane
     if (value < -1 || value > 1) return XS_ERR_ARG;
     c->trsv_prog = (int)value;
     c->ilu.trsv_prog = c->trsv_prog;
+    c->ilu.have_t = false;
   }
   else if (k == "trsv_gather") {   // 0 by factor width, 4 or 16 off-group entries per poll
     if (value != 0 && value != 4 && value != 16) return XS_ERR_ARG;
@@ -1008,22 +1017,64 @@ static int build_trsv_schedules(xs_ctx *c, const int *rp, const int *ci, const i
   return XS_OK;
 }
 
-// The row groups of a factor pattern (ILU(0) / IC(0) on A's pattern,
-// ParILUT's own), on the first solve that applies the factor by the exact
-// triangular solve (sweep counts < 0): a host pass over a copy of the
-// pattern.
-static int ensure_trsv_sched(xs_ctx *c, bool exact) {
-  xs_ilu &F = c->ilu;
-  if (!F.sched_pending || (!exact && c->lsweeps >= 0 && c->usweeps >= 0)) return XS_OK;
-  const int n = F.n, nnz = F.nnz;
-  std::vector<int> hrp(n + 1), hci(nnz), hdp(n);
+// values of the chains that hold earlier ones
+static int strip_values(xs_ctx *c, xs_strip &S, const double *lu) {
+  if (!S.ready || S.vals) return XS_OK;
+  xs_strip_values(c->stream, lu, S);
+  // the solve may run on another stream
   XS_HIP(hipStreamSynchronize(c->stream));
-  XS_HIP(hipMemcpy(hrp.data(), F.rp, sizeof(int) * (n + 1), hipMemcpyDeviceToHost));
-  XS_HIP(hipMemcpy(hci.data(), F.ci, sizeof(int) * nnz, hipMemcpyDeviceToHost));
-  XS_HIP(hipMemcpy(hdp.data(), F.dpos, sizeof(int) * n, hipMemcpyDeviceToHost));
-  const int rc = build_trsv_schedules(c, hrp.data(), hci.data(), hdp.data());
-  if (rc == XS_OK) F.sched_pending = false;
+  return xs_take_launch_guard() ? XS_ERR_STATE : XS_OK;
+}
+
+// chains of both triangles of a pattern (host copy; d_*: on the device), or
+// neither
+static int build_strips(xs_ctx *c, int n, const int *rp, const int *ci, const int *dpos,
+                        const int *d_rp, const int *d_ci, const int *d_dpos, xs_strip &L,
+                        xs_strip &U) {
+  xs_strip_plan pl, pu;
+  int rc = XS_OK;
+  if (xs_strip_analyse(n, rp, ci, dpos, false, pl) && xs_strip_analyse(n, rp, ci, dpos, true, pu) &&
+      ((rc = xs_strip_build(c->stream, n, d_rp, d_ci, d_dpos, false, pl, L)) ||
+       (rc = xs_strip_build(c->stream, n, d_rp, d_ci, d_dpos, true, pu, U)))) {
+    xs_strip_free(L);
+    xs_strip_free(U);
+    if (rc == XS_ERR_MEMORY) rc = XS_OK;   // the general solve needs less
+  }
+  L.tried = U.tried = true;
   return rc;
+}
+
+// What the exact triangular solves of a factor pattern (ILU(0) / IC(0) on A's
+// pattern, ParILUT's own) need, on the first solve that applies it by them
+// (sweep counts < 0): for the FP64 solves of one right-hand side
+// (NEED_CHAINS) the chains of a narrow factor, else, and for the other solves
+// (NEED_GROUPS), the row groups and their order; host passes over a copy of
+// the pattern.
+static int ensure_trsv_sched(xs_ctx *c, bool exact, int need) {
+  xs_ilu &F = c->ilu;
+  if (!exact && c->lsweeps >= 0 && c->usweeps >= 0) return XS_OK;
+  const bool chains = (need & NEED_CHAINS) && F.chains && F.trsv_prog != 1 && xs_ilu_gather(F) != 16;
+  auto need_groups = [&]() {
+    return F.sched_pending && ((need & NEED_GROUPS) || !(chains && F.sl.ready));
+  };
+  int rc = XS_OK;
+  if ((chains && !F.sl.tried) || need_groups()) {
+    const int n = F.n, nnz = F.nnz;
+    std::vector<int> hrp(n + 1), hci(nnz), hdp(n);
+    XS_HIP(hipStreamSynchronize(c->stream));
+    XS_HIP(hipMemcpy(hrp.data(), F.rp, sizeof(int) * (n + 1), hipMemcpyDeviceToHost));
+    XS_HIP(hipMemcpy(hci.data(), F.ci, sizeof(int) * nnz, hipMemcpyDeviceToHost));
+    XS_HIP(hipMemcpy(hdp.data(), F.dpos, sizeof(int) * n, hipMemcpyDeviceToHost));
+    if (chains && !F.sl.tried &&
+        (rc = build_strips(c, n, hrp.data(), hci.data(), hdp.data(), F.rp, F.ci, F.dpos, F.sl, F.su)))
+      return rc;
+    if (need_groups()) {
+      if ((rc = build_trsv_schedules(c, hrp.data(), hci.data(), hdp.data()))) return rc;
+      F.sched_pending = false;
+    }
+  }
+  if (chains && ((rc = strip_values(c, F.sl, F.lu)) || (rc = strip_values(c, F.su, F.lu)))) return rc;
+  return XS_OK;
 }
 
 // Update lists of the ParILU(0) / ParIC(0) sweeps (once per pattern, on
@@ -1373,6 +1424,8 @@ int xs_parilut_factor(xs_ctx *c) {
   F.sched_pending = false;
   F.nact = 0;
   F.tell_shape = false;   // a new pattern: the sweep copies are re-shaped
+  F.have_tp = false;
+  for (xs_strip *S : {&F.sl, &F.su, &F.tsl, &F.tsu}) xs_strip_free(*S);
   int rc;
   double *dtol = nullptr, *thr = nullptr;
   int *cnt = nullptr, *bsum = nullptr, *ovf = nullptr, *lrows = nullptr, *nlong = nullptr;
@@ -1565,6 +1618,7 @@ extern "C" int xs_pc_setup(xs_ctx *c) {
   if (xs_take_launch_guard()) rc = XS_ERR_STATE;
   if (rc == XS_OK) c->pc_ready = true;
   c->ilu.have_t = false;
+  for (xs_strip *S : {&c->ilu.sl, &c->ilu.su, &c->ilu.tsl, &c->ilu.tsu}) S->vals = false;
   c->mixed_ready = false;   // FP32 copies of A and of the factors are rebuilt
   c->tell_ready = c->tell32_ready = false;   // and the sweep copies of the factors
   return rc;
@@ -1852,7 +1906,7 @@ static int finish_solve(xs_ctx *c, int rc) {
 }
 
 // common checks and lazy set-up before a solve
-static int prepare_solve(xs_ctx *c) {
+static int prepare_solve(xs_ctx *c, bool block = false) {
   int rc;
   if (!c->mat_ready) return XS_ERR_STATE;
   if (c->ksp == XS_KSP_NONE) return XS_ERR_STATE;
@@ -1862,7 +1916,8 @@ static int prepare_solve(xs_ctx *c) {
   if (xs_pc_factored(c->pc) && (c->lsweeps >= 2 || c->usweeps >= 2) &&
       (rc = ensure_tri_ell(c)))
     return rc;
-  return ensure_trsv_sched(c);
+  if (!xs_pc_factored(c->pc)) return XS_OK;
+  return ensure_trsv_sched(c, false, block || c->precision == 1 ? NEED_GROUPS : NEED_CHAINS);
 }
 
 static int run_solve(xs_ctx *c, const double *d_b, double *d_x) {
@@ -1912,7 +1967,7 @@ extern "C" int xs_solve_device(xs_ctx *c, const double *d_rhs, double *d_sol) {
 // ---------------------------------------------------------------------------
 static int run_multi(xs_ctx *c, int k, const double *d_b, double *d_x, int layout) {
   int rc;
-  if ((rc = prepare_solve(c))) return rc;
+  if ((rc = prepare_solve(c, true))) return rc;
   if (c->precision != 0) {
     snprintf(xs_errbuf, sizeof(xs_errbuf), "block solve: FP64 only (precision 0)");
     return XS_ERR_UNSUPPORTED;
@@ -2039,6 +2094,9 @@ extern "C" double xs_get_time_ms(const xs_ctx *c, const char *phase) {
   if (!strcmp(phase, "spmv:dia")) return (c->use_ell && c->ell.dv) ? (double)c->ell.nd : 0.0;
   if (!strcmp(phase, "pc:dia")) return c->tell_ready ? (double)c->ilu.tl.nd : -1.0;
   if (!strcmp(phase, "parilu:dia")) return (double)c->ilu.pnd;
+  // chains of L's exact solve (0: the general solve, -1: not looked at yet)
+  if (!strcmp(phase, "trsv:chains"))
+    return !c->ilu.sl.tried ? -1.0 : xs_strip_used(c->ilu, c->ilu.sl) ? (double)c->ilu.sl.nchains : 0.0;
   // 1 when both sweep copies of the factors carry 16-bit offsets (-1: not built)
   if (!strcmp(phase, "pc:idx16"))
     return !c->tell_ready ? -1.0
@@ -2087,14 +2145,18 @@ int xs_build_transpose(xs_ctx *c) {
   return ensure_common(c);
 }
 
-int xs_build_factor_transpose(xs_ctx *c) {
+// transposed pattern of the factors, once per pattern: CSR, pivot positions
+// and, for its triangular solves, chains or row groups in level order (host,
+// from a copy)
+static int build_transposed_pattern(xs_ctx *c, bool chains) {
   xs_ilu &F = c->ilu;
-  if (F.have_t) return XS_OK;
   const int n = F.n, nnz = F.nnz;
   int rc;
   dfree(F.trp); dfree(F.tci); dfree(F.tdpos); dfree(F.tlu); dfree(F.tperm);
   dfree(F.tlgb); dfree(F.tugb); dfree(F.tlsched); dfree(F.tusched);
   F.tlgroups = F.tugroups = 0;
+  xs_strip_free(F.tsl);
+  xs_strip_free(F.tsu);
   if ((rc = dalloc(&F.trp, n + 1)) || (rc = dalloc(&F.tci, nnz)) || (rc = dalloc(&F.tdpos, n)) ||
       (rc = dalloc(&F.tlu, nnz)) || (rc = dalloc(&F.tperm, nnz)))
     return rc;
@@ -2103,31 +2165,49 @@ int xs_build_factor_transpose(xs_ctx *c) {
   if ((rc = device_transpose(c, n, nnz, F.ci, F.rowidx, F.trp, F.tci, F.tperm))) return rc;
   XS_HIP(hipMemsetAsync(c->d_int, 0, sizeof(int), c->stream));
   xs_pt_dpos(c->stream, n, F.trp, F.tci, F.tdpos, c->d_int);
-  // row groups and level order of the transposed triangular solves (host,
-  // from a copy of the transposed pattern)
   std::vector<int> trp(n + 1), tci(nnz), tdpos(n);
   XS_HIP(hipStreamSynchronize(c->stream));
   XS_HIP(hipMemcpy(trp.data(), F.trp, sizeof(int) * (n + 1), hipMemcpyDeviceToHost));
   XS_HIP(hipMemcpy(tci.data(), F.tci, sizeof(int) * nnz, hipMemcpyDeviceToHost));
   XS_HIP(hipMemcpy(tdpos.data(), F.tdpos, sizeof(int) * n, hipMemcpyDeviceToHost));
-  {
-    std::vector<int> gb, ord;
-    for (int part = 0; part < 2; ++part) {
-      const bool upper = part == 1;
-      trsv_groups(n, trp.data(), tci.data(), tdpos.data(), upper, gb);
-      const int G = (int)gb.size() - 1;
-      int *&dgb = upper ? F.tugb : F.tlgb;
-      if ((rc = dalloc(&dgb, (size_t)G + 1))) return rc;
-      XS_HIP(hipMemcpy(dgb, gb.data(), sizeof(int) * (G + 1), hipMemcpyHostToDevice));
-      (upper ? F.tugroups : F.tlgroups) = G;
-      if (!c->trsv_schedule) continue;
-      group_order(n, trp.data(), tci.data(), tdpos.data(), upper, gb, ord);
-      int *&ds = upper ? F.tusched : F.tlsched;
-      if ((rc = dalloc(&ds, (size_t)G))) return rc;
-      XS_HIP(hipMemcpy(ds, ord.data(), sizeof(int) * G, hipMemcpyHostToDevice));
-    }
+  if (chains && (rc = build_strips(c, n, trp.data(), tci.data(), tdpos.data(), F.trp, F.tci,
+                                   F.tdpos, F.tsl, F.tsu)))
+    return rc;
+  if (F.tsl.ready) return XS_OK;
+  std::vector<int> gb, ord;
+  for (int part = 0; part < 2; ++part) {
+    const bool upper = part == 1;
+    trsv_groups(n, trp.data(), tci.data(), tdpos.data(), upper, gb);
+    const int G = (int)gb.size() - 1;
+    int *&dgb = upper ? F.tugb : F.tlgb;
+    if ((rc = dalloc(&dgb, (size_t)G + 1))) return rc;
+    XS_HIP(hipMemcpy(dgb, gb.data(), sizeof(int) * (G + 1), hipMemcpyHostToDevice));
+    (upper ? F.tugroups : F.tlgroups) = G;
+    if (!c->trsv_schedule) continue;
+    group_order(n, trp.data(), tci.data(), tdpos.data(), upper, gb, ord);
+    int *&ds = upper ? F.tusched : F.tlsched;
+    if ((rc = dalloc(&ds, (size_t)G))) return rc;
+    XS_HIP(hipMemcpy(ds, ord.data(), sizeof(int) * G, hipMemcpyHostToDevice));
   }
-  xs_permute_vals(c->stream, nnz, F.tperm, F.lu, F.tlu);
+  return XS_OK;
+}
+
+int xs_build_factor_transpose(xs_ctx *c) {
+  xs_ilu &F = c->ilu;
+  if (F.have_t) return XS_OK;
+  int rc;
+  const bool chains = F.chains && F.trsv_prog != 1 && xs_ilu_gather(F) != 16;
+  // a pattern stays as it is over new values; what its solves need is built
+  // again when the options ask for the other form
+  if (!F.have_tp || (chains ? !F.tsl.tried : F.tlgb == nullptr)) {
+    F.have_tp = false;
+    if ((rc = build_transposed_pattern(c, chains))) return rc;
+    F.have_tp = true;
+  }
+  xs_permute_vals(c->stream, F.nnz, F.tperm, F.lu, F.tlu);
+  F.tsl.vals = F.tsu.vals = false;
+  if (chains && ((rc = strip_values(c, F.tsl, F.tlu)) || (rc = strip_values(c, F.tsu, F.tlu))))
+    return rc;
   XS_HIP(hipStreamSynchronize(c->stream));
   if (xs_take_launch_guard()) return XS_ERR_STATE;
   F.have_t = true;
@@ -2199,7 +2279,7 @@ extern "C" int xs_pc_apply(xs_ctx *c, const double *x, double *y, void *stream) 
   if (xs_pc_factored(c->pc) && (c->lsweeps >= 2 || c->usweeps >= 2) &&
       (rc = ensure_tri_ell(c)))
     return rc;
-  if ((rc = ensure_trsv_sched(c))) return rc;
+  if (xs_pc_factored(c->pc) && (rc = ensure_trsv_sched(c, false, NEED_CHAINS))) return rc;
   hipStream_t keep = c->stream;
   c->stream = pick(c, stream);
   xs_op_pc(c, x, y, xs_ctx_vec(c, XS_NWORK - 1), nullptr);
@@ -2248,7 +2328,7 @@ extern "C" int xs_pc_apply_multi(xs_ctx *c, int nrhs, const double *x, double *y
     case XS_PC_IC0: {
       if ((rc = xs_multi_reserve(c, nrhs, 1))) return rc;
       if ((c->lsweeps >= 2 || c->usweeps >= 2) && (rc = ensure_tri_ell(c))) return rc;
-      if ((rc = ensure_trsv_sched(c))) return rc;
+      if ((rc = ensure_trsv_sched(c, false, NEED_GROUPS))) return rc;
       xs_multi_ilu_apply(c, s, nrhs, x, y, xs_multi_vec(c, nrhs, 8), xs_multi_vec(c, nrhs, 9),
                          nullptr);
       break;
@@ -2265,7 +2345,7 @@ extern "C" int xs_trsv(xs_ctx *c, int which, const double *b, double *x, void *s
   int rc;
   if (!xs_pc_factored(c->pc)) return XS_ERR_STATE;
   if (!c->pc_ready && (rc = xs_pc_setup(c))) return rc;
-  if ((rc = ensure_trsv_sched(c, true))) return rc;   // an exact solve whatever the apply
+  if ((rc = ensure_trsv_sched(c, true, NEED_CHAINS))) return rc;   // an exact solve whatever the apply
   xs_fill_sentinel(pick(c, stream), x, c->A.n);
   if (which == 0) xs_trsv_lower(pick(c, stream), c->ilu, b, x, c->counters + 2, nullptr);
   else xs_trsv_upper(pick(c, stream), c->ilu, b, x, c->counters + 4, nullptr);

@@ -5,6 +5,8 @@
 #include <cstddef>
 #include <cstdint>
 
+#include "xs_strip.h"
+
 #define XS_BLOCK 256          // threads per workgroup for streaming kernels
 #define XS_WAVE 64            // CDNA wavefront
 #define XS_SPMV_LDS 4096      // products staged in LDS per CSR row block (32 KiB)
@@ -233,7 +235,17 @@ struct xs_ilu {
   double *tlu = nullptr;
   int *tlgb = nullptr, *tugb = nullptr, *tlsched = nullptr, *tusched = nullptr;
   int tlgroups = 0, tugroups = 0;
+  bool have_tp = false;     // the transposed pattern (and its groups) are current
+  // chains of the narrow triangles (L, U and of the transposed factors) for
+  // the FP64 solves of one right-hand side; used when `chains` is set
+  bool chains = true;
+  xs_strip sl, su, tsl, tsu;
 };
+
+// the triangle's solve runs over its chains
+inline bool xs_strip_used(const xs_ilu &F, const xs_strip &S) {
+  return F.chains && S.ready && S.vals && F.trsv_prog != 1;
+}
 
 // the gather width of a factor's triangular solves: the set one, else by width
 inline int xs_ilu_gather(const xs_ilu &F) {

@@ -1622,10 +1622,12 @@ static void trsv_launch(hipStream_t s, bool upper, int n, const int *rp, const i
 
 void xs_trsv_lower(hipStream_t s, const xs_ilu &F, const double *b, double *x, unsigned *tickets,
                    const xs_state *st) {
+  if (xs_strip_used(F, F.sl)) return xs_strip_solve(s, F.sl, false, nullptr, b, x, tickets, st);
   trsv_launch(s, false, F.n, F.rp, F.ci, F.lu, F.dpos, nullptr, b, x, tickets, xs_ilu_tsched(F, false), st);
 }
 void xs_trsv_upper(hipStream_t s, const xs_ilu &F, const double *b, double *x, unsigned *tickets,
                    const xs_state *st) {
+  if (xs_strip_used(F, F.su)) return xs_strip_solve(s, F.su, true, F.dinv, b, x, tickets, st);
   trsv_launch(s, true, F.n, F.rp, F.ci, F.lu, F.dpos, F.dinv, b, x, tickets, xs_ilu_tsched(F, true), st);
 }
 // Transposed factors (F^T = U^T | L^T on the transposed pattern): the lower
@@ -1633,6 +1635,7 @@ void xs_trsv_upper(hipStream_t s, const xs_ilu &F, const double *b, double *x, u
 // 64-row groups in solve order.
 void xs_trsv_lower_t(hipStream_t s, const xs_ilu &F, const double *b, double *x,
                      unsigned *tickets, const xs_state *st) {
+  if (xs_strip_used(F, F.tsl)) return xs_strip_solve(s, F.tsl, false, F.dinv, b, x, tickets, st);
   xs_tsched S;
   S.gb = F.tlgb;
   S.ngroups = F.tlgroups;
@@ -1644,6 +1647,7 @@ void xs_trsv_lower_t(hipStream_t s, const xs_ilu &F, const double *b, double *x,
 }
 void xs_trsv_upper_t(hipStream_t s, const xs_ilu &F, const double *b, double *x,
                      unsigned *tickets, const xs_state *st) {
+  if (xs_strip_used(F, F.tsu)) return xs_strip_solve(s, F.tsu, true, nullptr, b, x, tickets, st);
   xs_tsched S;
   S.gb = F.tugb;
   S.ngroups = F.tugroups;

@@ -52,6 +52,7 @@ struct xs_ctx {
   bool fuse_p = false;          // BiCGSTAB forms p inside the first L pass (slower when launched directly)
   int use_graph = -1;           // replay batches as HIP graphs: 1 all solves, 0 none, -1 k-RHS blocks
   bool trsv_schedule = true;    // SpTRSV groups in dependency-level order
+  bool trsv_chains = true;      // FP64 SpTRSV of narrow factors over chains of groups when possible
   int trsv_wg = 256;            // persistent workgroups of the SpTRSV
   int trsv_prog = -1;           // SpTRSV group mode (xs_tsched::prog), -1 = by factor width
   int trsv_gather = 0;          // SpTRSV gather width (4 or 16), 0 = by factor width
