@@ -333,3 +333,50 @@ def test_block_errors(dev):
         S.solve_multi(np.ones((256, 65)))
     assert e.value.status == xsolver_amd.XS_ERR_ARG
     S.close()
+
+
+ELL_EDGES = {  # name: (matrix, columns)
+    "runs_tail": (lambda: gen.convdiff3d(33), 32),      # 4-block runs, ragged last rows
+    "runs_16": (lambda: gen.poisson2d(401), 16),        # 16 rows a wave, 2 entries a lane
+    "runs_64": (lambda: gen.poisson2d(150), 64),        # 4 rows a wave
+    "wide_rows": (lambda: gen.lognormal27(13, seed=5), 32),   # 27 entries, 4 a lane
+    "wide_direct": (lambda: gen.lognormal27(14, seed=5), 16),  # too many to stage
+    "past_caches": (lambda: gen.poisson2d(512), 32),    # 64 MB: streamed results
+    "below": (lambda: gen.poisson2d(511), 32),
+    "past_caches_8": (lambda: gen.convdiff3d(102), 8),  # streamed, not staged
+    "few_blocks": (lambda: gen.poisson2d(13), 32),      # fewer than the XCDs
+}
+
+
+@pytest.mark.parametrize("name", list(ELL_EDGES))
+def test_multi_ell_edges(dev, name):
+    """Product and apply of the k-column ELL kernels where their row order,
+    staging and stores change, against those of single vectors bit for bit
+    (both sum a row in entry order; columns that are masked one by one are
+    test_block_per_column_masks')."""
+    import torch
+    make, k = ELL_EDGES[name]
+    A = make()
+    n = len(A[0]) - 1
+    say(f"[multi-ell] {name} n={n} k={k}")
+    B = np.random.default_rng(40).uniform(-1, 1, (n, k))
+    Bd = dev_tensor(B, dev)
+    Yd = torch.empty_like(Bd)
+    y1 = torch.empty(n, dtype=torch.float64, device=dev)
+    S = XSolver()
+    S.mat_setup(*A)
+    S.ksp_settype("bicgstab")
+    S.pc_settype("ilu0")
+    S.set_option("lsolve_sweeps", 3)
+    S.set_option("usolve_sweeps", 3)
+    S.pc_setup()
+    assert S.time_ms("spmv:kernel") == 2   # an ELL copy: entry order in both products
+    for multi, single in ((S.spmm, S.spmv), (S.pc_apply_multi, S.pc_apply)):
+        Yd.fill_(float("nan"))
+        multi(Bd, Yd, torch_stream())
+        for j in (0, 1, k // 2 - 1, k // 2, k - 1):
+            single(Bd[:, j].contiguous(), y1, torch_stream())
+            torch.cuda.synchronize()
+            assert torch.equal(Yd[:, j], y1), j
+        assert torch.isfinite(Yd).all()
+    S.close()

@@ -264,11 +264,13 @@ static bool ell_fits(const std::vector<int> &hrp) {
 // 16-bit column offsets beside the int32 columns of an ELL layout when every
 // entry is within XS_OFF16_MAX of its row (the kernels then read 2 instead of
 // 4 index bytes per entry); *co stays null otherwise.
-static int make_offsets(xs_ctx *c, int n, int ld, int W, const int *eci, short **co) {
+static int make_offsets(xs_ctx *c, int n, int ld, int W, const int *eci, short **co, int *far) {
   dfree(*co);
+  *far = 0;
   if (W == 0 || n == 0) return XS_OK;
   const int m = xs_ell_max_offset(c->stream, n, ld, W, eci, c->d_int);
   if (m < 0) return XS_ERR_DEVICE;
+  *far = m;
   if (m > XS_OFF16_MAX) return XS_OK;
   int rc;
   if ((rc = dalloc(co, (size_t)W * ld))) return rc;
@@ -288,7 +290,7 @@ static int make_ell(xs_ctx *c) {
   if ((rc = dalloc(&c->ell.ci, (size_t)W * c->ell.ld))) return rc;
   if ((rc = dalloc(&c->ell.v, (size_t)W * c->ell.ld))) return rc;
   xs_build_ell(c->stream, A, W, c->ell);
-  if ((rc = make_offsets(c, A.n, c->ell.ld, W, c->ell.ci, &c->ell.co))) return rc;
+  if ((rc = make_offsets(c, A.n, c->ell.ld, W, c->ell.ci, &c->ell.co, &c->ell.far))) return rc;
   // diagonal slots for the FP64 SpMV when A has few distinct offsets
   if (!c->spmv_dia) return XS_OK;
   xs_dia_offs off{};
@@ -1721,7 +1723,7 @@ static int ensure_tri_ell(xs_ctx *c) {
   if (!F.tell_shape) {   // offsets and group widths depend on the pattern only
     for (int part = 0; part < 2; ++part) {
       xs_tell &E = part ? F.tu : F.tl;
-      if ((rc = make_offsets(c, F.n, E.ld, E.W, E.ci, &E.co))) return rc;
+      if ((rc = make_offsets(c, F.n, E.ld, E.W, E.ci, &E.co, &E.far))) return rc;
       dfree(E.ww);
       if ((rc = dalloc(&E.ww, ((size_t)F.n + XS_WAVE - 1) / XS_WAVE))) return rc;
       xs_tri_wave_widths(c->stream, F, part == 1, E.ww);

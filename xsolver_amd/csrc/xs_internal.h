@@ -108,6 +108,7 @@ struct xs_ell {         // column-major slabs: v[k * ld + row], width W
   int *ci = nullptr;
   double *v = nullptr;
   short *co = nullptr;  // column - row as 16 bits (when every entry fits), else null
+  int far = 0;          // largest |column - row|
   // diagonal-slot copy (nd > 0): dv[k * ld + row] = a(row, row + doff.o[k])
   // or 0 where that entry is absent, the offsets ascending (the slots are in
   // column order, as the ELL rows); null when the matrix has more offsets
@@ -133,6 +134,7 @@ struct xs_tell {
   void *vlo = nullptr;       // values for the mixed inner solver (factor storage type)
   size_t vlo_bytes = 0;      // allocated bytes of vlo
   short *co = nullptr;       // column - row as 16 bits, XS_OFF16_PAD = padding
+  int far = 0;               // largest |column - row|
   int *ww = nullptr;         // per 64-row group (rows 64g ..): its longest row, the
                              // slab count the sweeps walk for those rows
   double *vs = nullptr;      // U only: u_ij / u_jj, the values of the first two

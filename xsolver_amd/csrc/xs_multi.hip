@@ -233,50 +233,152 @@ __device__ __forceinline__ void ell_batch(int i, int k0, int ld, int W, const in
   }
 }
 
-// SpMM over the ELL copy of A, CW adjacent columns per thread (k / CW
-// threads per row): the row's slab entries are loaded once per CW columns
-// and each gather moves CW contiguous values.  Per column the entry-order
+// Row blocks of the k-column ELL kernels, dealt to the XCDs (workgroup b runs
+// on XCD b % 8).  The vectors are too large for an L2 to hold a band of rows
+// (7-point 128^3 grid, 32 columns: 4 MB a plane), so what decides the traffic
+// between the L2s and memory is how often a row of X is fetched: with blocks
+// dealt one by one each XCD sees an eighth of every line and fetches its
+// neighbours in y and z again, five times X per product.  Dealt in runs of
+// `run` blocks, an eighth of the band (the largest |column - row|), an XCD
+// keeps to the same eighth of each plane: the neighbours in y are its own, and
+// those in z it has had one band ago, 0.5 MB.  What is left after the whole
+// bands is dealt one by one.  (Runs against blocks one by one: 75^3, 32 columns:
+// product 51 against 83 us; 120^3: 338 against 407.)
+struct xs_mmap {
+  int run, nblk, full;   // blocks of a run, of all rows, runs per XCD times run
+  bool nt;               // results past the caches (the kernels' NT)
+};
+__device__ __forceinline__ int mmap_block(const xs_mmap &M, int t, int xcd) {
+  if (t >= M.full) return t * XS_NXCD + xcd;
+  const int q = t / M.run;
+  return (q * XS_NXCD + xcd) * M.run + (t - q * M.run);
+}
+
+typedef double d2v __attribute__((ext_vector_type(2)));
+// CW values of a row to its columns jc(0) .. jc(CW - 1), those that are live
+template <int CW, bool NT, class J>
+__device__ __forceinline__ void mstore(double *row, const double (&y)[CW], const bool (&live)[CW], J jc) {
+  if (CW == 1) {
+    if (live[0]) row[jc(0)] = y[0];
+    return;
+  }
+#pragma unroll
+  for (int h = 0; h < CW; h += 2) {
+    if (live[h] && live[(h + 1) % CW]) {
+      const d2v v = {y[h], y[(h + 1) % CW]};
+      if (NT) __builtin_nontemporal_store(v, reinterpret_cast<d2v *>(row + jc(h)));
+      else *reinterpret_cast<d2v *>(row + jc(h)) = v;
+    }
+    else if (live[h]) row[jc(h)] = y[h];
+    else if (live[(h + 1) % CW]) row[jc(h + 1)] = y[(h + 1) % CW];
+  }
+}
+
+// The slab entries of a wave's 64 / L rows, EN to a lane: loaded a step ahead,
+// each by one lane, and handed to the L threads of its row through the wave's
+// part of LDS (LDS operations of a wave run in order).  Loaded by every thread
+// that needs them they were half of the kernel's load instructions (128^3, 32
+// columns, apply of 2 x 3 sweeps: 1337 us without, 1253 with).
+struct __align__(16) mentry {
+  double a;
+  int c, pad;
+};
+template <bool O16, int EN>
+struct mstage {
+  int c[EN ? EN : 1];
+  double a[EN ? EN : 1];
+  __device__ __forceinline__ void load(int i0, int lrw, int n, int ld, int W, const int *__restrict__ eci,
+                                       const short *__restrict__ eco, const double *__restrict__ ev) {
+    const int lane = threadIdx.x & (XS_WAVE - 1);
+#pragma unroll
+    for (int e = 0; e < EN; ++e) {
+      const int q = (e * XS_WAVE + lane) >> lrw, r = i0 + (lane & ((1 << lrw) - 1));
+      c[e] = -1;
+      a[e] = 0.0;
+      if (q < W && r < n) {
+        const size_t p = (size_t)q * ld + r;
+        const int o = O16 ? (int)eco[p] : eci[p];
+        a[e] = ev[p];
+        c[e] = O16 ? (o == XS_OFF16_PAD ? -1 : r + o) : o;
+      }
+    }
+  }
+  __device__ __forceinline__ void put(mentry *buf) const {
+    const int lane = threadIdx.x & (XS_WAVE - 1);
+#pragma unroll
+    for (int e = 0; e < EN; ++e) {
+      buf[e * XS_WAVE + lane].a = a[e];
+      buf[e * XS_WAVE + lane].c = c[e];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+};
+
+// SpMM over the ELL copy of A, CW columns per thread (k / CW threads
+// per row), in pairs k / 2 apart: the row's slab entries are loaded once per
+// CW columns, and the lanes of a load or store of 16 bytes are contiguous.
+// (Four adjacent columns a thread, stored one by one, were 8 write requests of
+// L2 per line.)  Bound by memory where the vectors exceed the caches.  7-point
+// 128^3, 32 columns: 520 -> 376 us (two vectors at 2.9 TB/s), 75^3: 81 -> 49.  Per column the entry-order
 // sum of k_mspmm.  Same epilogues; the workgroup's column sums go through
 // LDS (rows in order) to the shared cross-workgroup combine.
-template <int EPI, bool O16, int CW>
+template <int EPI, bool O16, int CW, bool NT, int EN>
 __global__ __launch_bounds__(XS_BLOCK) void k_mspmm_ell(
     int n, int k, int ld, int W, const int *__restrict__ eci, const short *__restrict__ eco,
     const double *__restrict__ ev, const double *__restrict__ X, double *__restrict__ Y,
-    const double *__restrict__ B, const double *__restrict__ Wv, xs_mred R, const xs_mstate *ms) {
+    const double *__restrict__ B, const double *__restrict__ Wv, xs_mmap M, xs_mred R,
+    const xs_mstate *ms) {
   if (ms && ms->all) return;
   constexpr int NV = (EPI == EPI_DOT2) ? 2 : 1;
   const int L = k / CW, per = XS_BLOCK / L;
-  const int g = threadIdx.x % L, rl = threadIdx.x / L, j0 = g * CW;
+  const int g = threadIdx.x % L, rl = threadIdx.x / L;
+  // this thread's c-th column
+  auto jc = [&](int c) { return CW == 1 ? g : (c / 2) * 2 * L + 2 * g + (c & 1); };
   bool live[CW];
   bool any = false;
 #pragma unroll
   for (int c = 0; c < CW; ++c) {
-    live[c] = rl < per && !(ms && ms->done[j0 + c]);
+    live[c] = rl < per && !(ms && ms->done[jc(c)]);
     any |= live[c];
   }
   double acc[NV][CW];
 #pragma unroll
   for (int c = 0; c < CW; ++c)
     for (int q = 0; q < NV; ++q) acc[q][c] = 0.0;
-  if (any) {
-    // the first slab batch of the thread's next row is loaded while the
-    // current row's gathers are in flight
-    const int stride = (int)gridDim.x * per;
-    int i = (int)blockIdx.x * per + rl;
+  __shared__ mentry stage[EN ? EN * XS_BLOCK : 1];
+  mentry *const sbuf = stage + (threadIdx.x / XS_WAVE) * (EN * XS_WAVE);
+  const int lrw = EN ? 31 - __clz(XS_WAVE / L) : 0, sr = EN ? (threadIdx.x & (XS_WAVE - 1)) / L : 0;
+  mstage<O16, EN> ahead;
+  if (EN > 0 || any) {
+    // the slab entries of the next step (the first batch of the thread's next
+    // row) are loaded while the current row's gathers are in flight
+    const int step = (int)gridDim.x / XS_NXCD, xcd = blockIdx.x % XS_NXCD;
+    int t = (int)blockIdx.x / XS_NXCD, i = mmap_block(M, t, xcd) * per + rl;
     int ncol[4];
     double na[4];
-    if (i < n) ell_batch<O16>(i, 0, ld, W, eci, eco, ev, ncol, na);
-    for (; i < n; i += stride) {
+    if (EN > 0) ahead.load(i - sr, lrw, n, ld, W, eci, eco, ev);
+    else if (i < n) ell_batch<O16>(i, 0, ld, W, eci, eco, ev, ncol, na);
+    while (i - sr < n) {   // EN: the same for a whole wave (sr is 0 otherwise)
+      t += step;
+      const int inext = t < M.nblk ? mmap_block(M, t, xcd) * per + rl : n + sr;
+      if (EN > 0) {
+        ahead.put(sbuf);
+        if (inext - sr < n) ahead.load(inext - sr, lrw, n, ld, W, eci, eco, ev);
+        if (i >= n || !any) {
+          i = inext;
+          continue;
+        }
+      }
       // the epilogue's operand row (B or W), loaded before the gathers
       double ep[CW];
 #pragma unroll
       for (int c = 0; c < CW; ++c) ep[c] = 0.0;
       if (EPI != EPI_Y) {
-        const double2 *src = reinterpret_cast<const double2 *>(
-            (EPI == EPI_BMAXN ? B : Wv) + (size_t)i * k + j0);
+        const double *src = (EPI == EPI_BMAXN ? B : Wv) + (size_t)i * k;
 #pragma unroll
         for (int h = 0; h < CW / 2; ++h) {
-          const double2 t = src[h];
+          const double2 t = *reinterpret_cast<const double2 *>(src + jc(2 * h));
           ep[2 * h] = t.x;
           ep[2 * h + 1] = t.y;
         }
@@ -287,10 +389,17 @@ __global__ __launch_bounds__(XS_BLOCK) void k_mspmm_ell(
       for (int k0 = 0; k0 < W; k0 += 4) {
         int col[4];
         double a[4];
-        if (k0 == 0) {
+        if (EN > 0) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const mentry m = sbuf[min(k0 + q, W - 1) << lrw | sr];
+            col[q] = k0 + q < W ? m.c : -1;
+            a[q] = m.a;
+          }
+        } else if (k0 == 0) {
 #pragma unroll
           for (int q = 0; q < 4; ++q) { col[q] = ncol[q]; a[q] = na[q]; }
-          if (i + stride < n) ell_batch<O16>(i + stride, 0, ld, W, eci, eco, ev, ncol, na);
+          if (inext < n) ell_batch<O16>(inext, 0, ld, W, eci, eco, ev, ncol, na);
         } else {
           ell_batch<O16>(i, k0, ld, W, eci, eco, ev, col, a);
         }
@@ -298,10 +407,10 @@ __global__ __launch_bounds__(XS_BLOCK) void k_mspmm_ell(
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           if (col[q] >= 0) {
-            const double2 *src = reinterpret_cast<const double2 *>(X + (size_t)col[q] * k + j0);
+            const double *src = X + (size_t)col[q] * k;
 #pragma unroll
             for (int h = 0; h < CW / 2; ++h) {
-              const double2 t = src[h];
+              const double2 t = *reinterpret_cast<const double2 *>(src + jc(2 * h));
               xv[q][2 * h] = t.x;
               xv[q][2 * h + 1] = t.y;
             }
@@ -316,20 +425,17 @@ __global__ __launch_bounds__(XS_BLOCK) void k_mspmm_ell(
 #pragma unroll
             for (int c = 0; c < CW; ++c) s[c] += a[q] * xv[q][c];
       }
+      double y[CW];
 #pragma unroll
       for (int c = 0; c < CW; ++c) {
+        y[c] = EPI == EPI_BMAXN ? ep[c] - s[c] : s[c];
         if (!live[c]) continue;
-        const size_t p = (size_t)i * k + j0 + c;
-        if (EPI == EPI_BMAXN) {
-          const double t = ep[c] - s[c];
-          Y[p] = t;
-          acc[0][c] += t * t;
-        } else {
-          Y[p] = s[c];
-          if (EPI == EPI_DOT1 || EPI == EPI_DOT2) acc[0][c] += ep[c] * s[c];
-          if (EPI == EPI_DOT2) acc[NV - 1][c] += s[c] * s[c];
-        }
+        if (EPI == EPI_BMAXN) acc[0][c] += y[c] * y[c];
+        if (EPI == EPI_DOT1 || EPI == EPI_DOT2) acc[0][c] += ep[c] * y[c];
+        if (EPI == EPI_DOT2) acc[NV - 1][c] += y[c] * y[c];
       }
+      mstore<CW, NT>(Y + (size_t)i * k, y, live, jc);
+      i = inext;
     }
   }
   if (EPI == EPI_Y) return;
@@ -338,7 +444,7 @@ __global__ __launch_bounds__(XS_BLOCK) void k_mspmm_ell(
   if (rl < per)
 #pragma unroll
     for (int c = 0; c < CW; ++c)
-      for (int q = 0; q < NV; ++q) cs[q][rl * k + j0 + c] = acc[q][c];
+      for (int q = 0; q < NV; ++q) cs[q][rl * k + jc(c)] = acc[q][c];
   __syncthreads();
   double bs[NV];
   for (int q = 0; q < NV; ++q) {
@@ -706,12 +812,12 @@ static inline int mgrid_flat(size_t m) {
   return g < 1 ? 1 : (int)g;
 }
 // k-column Jacobi sweep of a factor over its ELL copy (one pass, columns
-// interleaved): CW adjacent columns per thread, k / CW threads per row; the
-// row's slab entries are loaded once per CW columns and each gather moves CW
-// contiguous values.  Per column the arithmetic of k_tri_sweep_ell (FUSED:
+// interleaved): CW columns per thread, k / CW threads per row, in pairs as
+// k_mspmm_ell's, the same staging and the same order of rows (7-point 128^3,
+// 32 columns, 3 + 3 sweeps: 1610 -> 1169 us, 4.6 TB/s).  Per column the arithmetic of k_tri_sweep_ell (FUSED:
 // sweeps 1 and 2 from zero), so every column equals the single right-hand
 // side sweep.
-template <bool UPPER, bool FUSED, bool O16, int CW>
+template <bool UPPER, bool FUSED, bool O16, int CW, bool NT, int EN>
 __global__ __launch_bounds__(XS_BLOCK) void k_msweep_ell(int n, int k, int ld, int W,
                                                          const int *__restrict__ eci,
                                                          const short *__restrict__ eco,
@@ -720,49 +826,66 @@ __global__ __launch_bounds__(XS_BLOCK) void k_msweep_ell(int n, int k, int ld, i
                                                          const double *__restrict__ dinv,
                                                          const double *__restrict__ B,
                                                          const double *__restrict__ Yo,
-                                                         double *__restrict__ Yn,
+                                                         double *__restrict__ Yn, xs_mmap M,
                                                          const xs_mstate *ms) {
   if (ms && ms->all) return;
   const int L = k / CW, per = XS_BLOCK / L;
-  const int g = threadIdx.x % L, rl = threadIdx.x / L, j0 = g * CW;
+  const int g = threadIdx.x % L, rl = threadIdx.x / L;
+  // this thread's c-th column
+  auto jc = [&](int c) { return CW == 1 ? g : (c / 2) * 2 * L + 2 * g + (c & 1); };
   if (rl >= per) return;
   bool live[CW];
   bool any = false;
 #pragma unroll
   for (int c = 0; c < CW; ++c) {
-    live[c] = !(ms && ms->done[j0 + c]);
+    live[c] = !(ms && ms->done[jc(c)]);
     any |= live[c];
   }
-  if (!any) return;
-  // CW contiguous values of row r of an interleaved block
+  if (EN == 0 && !any) return;
+  __shared__ mentry stage[EN ? EN * XS_BLOCK : 1];
+  mentry *const sbuf = stage + (threadIdx.x / XS_WAVE) * (EN * XS_WAVE);
+  const int lrw = EN ? 31 - __clz(XS_WAVE / L) : 0, sr = EN ? (threadIdx.x & (XS_WAVE - 1)) / L : 0;
+  mstage<O16, EN> ahead;
+  // this thread's values of row r of an interleaved block
   auto load = [&](const double *base, int r, double (&out)[CW]) {
-    const double *src = base + (size_t)r * k + j0;
+    const double *src = base + (size_t)r * k;
     if (CW == 1) {
-      out[0] = src[0];
+      out[0] = src[jc(0)];
     } else {
 #pragma unroll
       for (int h = 0; h < CW / 2; ++h) {
-        const double2 t = reinterpret_cast<const double2 *>(src)[h];
+        const double2 t = *reinterpret_cast<const double2 *>(src + jc(2 * h));
         out[2 * h] = t.x;
         out[2 * h + 1] = t.y;
       }
     }
   };
-  // the first slab batch of the thread's next row is loaded while the
-  // current row's gathers are in flight
-  const int stride = (int)gridDim.x * per;
-  int i = (int)blockIdx.x * per + rl;
+  // the slab entries of the next step (the first batch of the thread's next
+  // row) are loaded while the current row's gathers are in flight
+  const int step = (int)gridDim.x / XS_NXCD, xcd = blockIdx.x % XS_NXCD;
+  int t = (int)blockIdx.x / XS_NXCD, i = mmap_block(M, t, xcd) * per + rl;
   int ncol[4];
   double na[4];
-  if (i < n) ell_batch<O16>(i, 0, ld, W, eci, eco, ev, ncol, na);
-  for (; i < n; i += stride) {
+  if (EN > 0) ahead.load(i - sr, lrw, n, ld, W, eci, eco, ev);
+  else if (i < n) ell_batch<O16>(i, 0, ld, W, eci, eco, ev, ncol, na);
+  while (i - sr < n) {   // EN: the same for a whole wave (sr is 0 otherwise)
+    t += step;
+    const int inext = t < M.nblk ? mmap_block(M, t, xcd) * per + rl : n + sr;
+    if (EN > 0) {
+      ahead.put(sbuf);
+      if (inext - sr < n) ahead.load(inext - sr, lrw, n, ld, W, eci, eco, ev);
+      if (i >= n || !any) {
+        i = inext;
+        continue;
+      }
+    }
     // this row's first batch; the next row's is loaded now, whether or not
     // this row walks its slabs
     int col0[4];
     double a0[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) { col0[q] = ncol[q]; a0[q] = na[q]; }
-    if (i + stride < n) ell_batch<O16>(i + stride, 0, ld, W, eci, eco, ev, ncol, na);
+    if (EN == 0 && inext < n) ell_batch<O16>(inext, 0, ld, W, eci, eco, ev, ncol, na);
     double bi[CW];
     load(B, i, bi);
     const double di = UPPER ? dinv[i] : 1.0;
@@ -774,7 +897,14 @@ __global__ __launch_bounds__(XS_BLOCK) void k_msweep_ell(int n, int k, int ld, i
     for (int k0 = 0; k0 < Wi; k0 += 4) {
       int col[4];
       double a[4];
-      if (k0 == 0) {
+      if (EN > 0) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const mentry m = sbuf[min(k0 + q, W - 1) << lrw | sr];
+          col[q] = k0 + q < W ? m.c : -1;
+          a[q] = m.a;
+        }
+      } else if (k0 == 0) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) { col[q] = col0[q]; a[q] = a0[q]; }
       } else {
@@ -801,8 +931,9 @@ __global__ __launch_bounds__(XS_BLOCK) void k_msweep_ell(int n, int k, int ld, i
           for (int c = 0; c < CW; ++c) r[c] += a[q] * y[q][c];
     }
 #pragma unroll
-    for (int c = 0; c < CW; ++c)
-      if (live[c]) Yn[(size_t)i * k + j0 + c] = UPPER ? di * (bi[c] - r[c]) : bi[c] - r[c];
+    for (int c = 0; c < CW; ++c) r[c] = UPPER ? di * (bi[c] - r[c]) : bi[c] - r[c];
+    mstore<CW, NT>(Yn + (size_t)i * k, r, live, jc);
+    i = inext;
   }
 }
 
@@ -855,24 +986,51 @@ static int resident_blocks(const void *kernel) {
   return r;
 }
 
-static dim3 ell_grid(const void *kernel, int n, int per) {
-  long g = ((long)n + per - 1) / per;
-  const long cap = std::min(XS_MGRID, resident_blocks(kernel));
-  if (g > cap) g = cap;
-  return dim3(g < 1 ? 1 : (unsigned)g);
+// Row blocks of `per` rows dealt in runs of an eighth of the band where there
+// are at least MAP_BANDS of them (fewer leave nothing to come back to).
+#define MAP_BANDS 4
+// Results of 64 MB and more are not in a cache when the next pass reads them:
+// stored past it they leave X its place, if a store fills whole pieces of a line
+// (100^3, 16 columns: product 72 against 109 us; 64^3, 8 columns, 17 MB: 16
+// against 14.5, and 4 columns, 32-byte pieces: apply 199 against 192).
+#define MAP_NT_BYTES (64u << 20)
+static xs_mmap ell_map(int n, int k, int per, int far) {
+  xs_mmap M{1, (n + per - 1) / per, 0, k >= 8 && (size_t)n * k * sizeof(double) >= MAP_NT_BYTES};
+  const long run = (far + XS_NXCD * (long)per / 2) / (XS_NXCD * (long)per);
+  if (run >= 1 && run * XS_NXCD * MAP_BANDS <= M.nblk) M.run = (int)run;
+  M.full = M.nblk / (XS_NXCD * M.run) * M.run;
+  return M;
+}
+// A multiple of the XCDs.  With staged slab entries four workgroups a CU have
+// enough loads in flight, and the fewer rows under way leave the L2s more of
+// the last band: 128^3, 32 columns: product 376 us with 1024, 433 with all
+// that fit, 443 with 512; without staging (8 columns) 133 and 115.
+#define MAP_STAGED_GRID 1024
+static dim3 ell_grid(const void *kernel, const xs_mmap &M, bool staged) {
+  const int cap = std::min(staged ? MAP_STAGED_GRID : XS_MGRID, resident_blocks(kernel)) / XS_NXCD * XS_NXCD;
+  const int g = (M.nblk + XS_NXCD - 1) / XS_NXCD * XS_NXCD;
+  return dim3(std::max(XS_NXCD, std::min(g, cap)));
+}
+
+// slab entries a lane stages (0: every thread loads its own): rows must not
+// straddle waves, at least four threads share an entry, and the entries ahead
+// must fit in registers
+static int ell_stage(int W, int L) {
+  if (L < 4 || L > XS_WAVE || (L & (L - 1)) || W == 0) return 0;
+  const int e = (W * (XS_WAVE / L) + XS_WAVE - 1) / XS_WAVE;
+  return e == 1 ? 1 : e == 2 ? 2 : e <= 4 ? 4 : 0;
 }
 
 // ELL SpMM: k even, every vector 16-byte aligned (checked by the caller)
-template <bool O16, int CW>
-static void mspmm_ell_launch(hipStream_t s, const xs_ell &E, int k, const double *X, double *Y,
-                             int epi, const double *B, const double *W, const xs_mred &R,
+template <bool O16, int CW, bool NT, int EN>
+static void mspmm_ell_launch(hipStream_t s, const xs_ell &E, int k, const xs_mmap &M, const double *X,
+                             double *Y, int epi, const double *B, const double *W, const xs_mred &R,
                              const xs_mstate *ms) {
-  const int per = XS_BLOCK / (k / CW);
   const dim3 blk(XS_BLOCK);
 #define XS_MSPMM_ELL(EP)                                                                        \
-  hipLaunchKernelGGL((k_mspmm_ell<EP, O16, CW>),                                               \
-                     ell_grid(reinterpret_cast<const void *>(&k_mspmm_ell<EP, O16, CW>), E.n, per), \
-                     blk, 0, s, E.n, k, E.ld, E.W, E.ci, E.co, E.v, X, Y, B, W, R, ms)
+  hipLaunchKernelGGL((k_mspmm_ell<EP, O16, CW, NT, EN>),                                       \
+                     ell_grid(reinterpret_cast<const void *>(&k_mspmm_ell<EP, O16, CW, NT, EN>), M, EN > 0), \
+                     blk, 0, s, E.n, k, E.ld, E.W, E.ci, E.co, E.v, X, Y, B, W, M, R, ms)
   switch (epi) {
     case EPI_Y: XS_MSPMM_ELL(EPI_Y); break;
     case EPI_DOT1: XS_MSPMM_ELL(EPI_DOT1); break;
@@ -900,13 +1058,24 @@ void xs_mspmm_ell(hipStream_t s, const xs_ell &E, int k, const double *X, double
   XS_GUARD(!(epi == EPI_DOT1 || epi == EPI_DOT2) || W);
   const xs_mred R = red ? *red : xs_mred{};
   const bool o16 = E.co != nullptr;
-  if (k % 4 == 0 && cw != 2) {
-    if (o16) mspmm_ell_launch<true, 4>(s, E, k, X, Y, epi, B, W, R, ms);
-    else mspmm_ell_launch<false, 4>(s, E, k, X, Y, epi, B, W, R, ms);
-  } else {
-    if (o16) mspmm_ell_launch<true, 2>(s, E, k, X, Y, epi, B, W, R, ms);
-    else mspmm_ell_launch<false, 2>(s, E, k, X, Y, epi, B, W, R, ms);
-  }
+  const int c = k % 4 == 0 && cw != 2 ? 4 : 2;
+  const xs_mmap M = ell_map(E.n, k, XS_BLOCK / (k / c), E.far);
+  const int en = c == 4 ? ell_stage(E.W, k / 4) : 0;
+#define XS_MSP(O, C, N, EN) mspmm_ell_launch<O, C, N, EN>(s, E, k, M, X, Y, epi, B, W, R, ms)
+#define XS_MSN(O, C, EN) do { if (M.nt) XS_MSP(O, C, true, EN); else XS_MSP(O, C, false, EN); } while (0)
+#define XS_MSC(O)                                                                              \
+  do {                                                                                         \
+    if (c == 2) XS_MSN(O, 2, 0);                                                               \
+    else if (en == 1) XS_MSN(O, 4, 1);                                                         \
+    else if (en == 2) XS_MSN(O, 4, 2);                                                         \
+    else if (en == 4) XS_MSN(O, 4, 4);                                                         \
+    else XS_MSN(O, 4, 0);                                                                      \
+  } while (0)
+  if (o16) XS_MSC(true);
+  else XS_MSC(false);
+#undef XS_MSC
+#undef XS_MSN
+#undef XS_MSP
 }
 
 void xs_mdot(hipStream_t s, int n, int k, const double *a, const double *b, const double *c,
@@ -965,18 +1134,29 @@ void xs_msweep_ell(hipStream_t s, const xs_tell &E, int n, int k, bool upper, bo
   const bool al = ((reinterpret_cast<uintptr_t>(B) | reinterpret_cast<uintptr_t>(Yo) |
                     reinterpret_cast<uintptr_t>(Yn)) & 15) == 0;
   const int cw = !al ? 1 : (k % 4 == 0 ? 4 : (k % 2 == 0 ? 2 : 1));
-  const int per = XS_BLOCK / (k / cw);
+  const xs_mmap M = ell_map(n, k, XS_BLOCK / (k / cw), E.far);
+  const int en = cw == 4 ? ell_stage(E.W, k / 4) : 0;
   const dim3 blk(XS_BLOCK);
-#define XS_MSK(U, FU, O, C)                                                                    \
-  hipLaunchKernelGGL((k_msweep_ell<U, FU, O, C>),                                             \
-                     ell_grid(reinterpret_cast<const void *>(&k_msweep_ell<U, FU, O, C>), n, per), \
-                     blk, 0, s, n, k, E.ld, E.W, E.ci, E.co, ev, E.ww, dinv, B, Yo, Yn, ms)
-#define XS_MSC(U, FU, O) do { if (cw == 4) XS_MSK(U, FU, O, 4); else if (cw == 2) XS_MSK(U, FU, O, 2); else XS_MSK(U, FU, O, 1); } while (0)
+#define XS_MSK(U, FU, O, C, N, EN)                                                             \
+  hipLaunchKernelGGL((k_msweep_ell<U, FU, O, C, N, EN>),                                      \
+                     ell_grid(reinterpret_cast<const void *>(&k_msweep_ell<U, FU, O, C, N, EN>), M, EN > 0), \
+                     blk, 0, s, n, k, E.ld, E.W, E.ci, E.co, ev, E.ww, dinv, B, Yo, Yn, M, ms)
+#define XS_MSN(U, FU, O, C, EN) do { if (M.nt) XS_MSK(U, FU, O, C, true, EN); else XS_MSK(U, FU, O, C, false, EN); } while (0)
+#define XS_MSC(U, FU, O)                                                                       \
+  do {                                                                                         \
+    if (cw == 1) XS_MSK(U, FU, O, 1, false, 0);                                                \
+    else if (cw == 2) XS_MSN(U, FU, O, 2, 0);                                                  \
+    else if (en == 1) XS_MSN(U, FU, O, 4, 1);                                                  \
+    else if (en == 2) XS_MSN(U, FU, O, 4, 2);                                                  \
+    else if (en == 4) XS_MSN(U, FU, O, 4, 4);                                                  \
+    else XS_MSN(U, FU, O, 4, 0);                                                               \
+  } while (0)
 #define XS_MSE(U, FU) do { if (E.co) XS_MSC(U, FU, true); else XS_MSC(U, FU, false); } while (0)
   if (upper) { if (fused) XS_MSE(true, true); else XS_MSE(true, false); }
   else { if (fused) XS_MSE(false, true); else XS_MSE(false, false); }
 #undef XS_MSE
 #undef XS_MSC
+#undef XS_MSN
 #undef XS_MSK
 }
 
