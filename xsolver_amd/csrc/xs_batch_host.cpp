@@ -113,9 +113,11 @@ extern "C" int xs_batch_create(xs_batch **out, int nsys, const int *sys_ptr, con
   BT_CHK(hipMemcpy(bt->rp, rowptr, sizeof(int) * (n + 1), hipMemcpyHostToDevice));
   BT_CHK(hipMemcpy(bt->ci, colidx, sizeof(int) * nnz, hipMemcpyHostToDevice));
   BT_CHK(hipMemcpy(bt->v, val, sizeof(double) * nnz, hipMemcpyHostToDevice));
-  // the systems' diagonal offsets, and slots when every system has few
+  // the systems' diagonal offsets, and slots when every system has few (the
+  // flags are cleared on the stream of the kernels that set them: it does not
+  // wait for the null stream)
   int stat[2] = {0, 0};
-  BT_CHK(hipMemset(bt->bad, 0, 2 * sizeof(int)));
+  BT_CHK(hipMemsetAsync(bt->bad, 0, 2 * sizeof(int), bt->stream));
   xs_batch_offsets(bt->stream, nsys, bt->sys_ptr, bt->rp, bt->ci, bt->off, bt->bad);
   BT_CHK(hipMemcpyAsync(stat, bt->bad, sizeof(stat), hipMemcpyDeviceToHost, bt->stream));
   BT_CHK(hipStreamSynchronize(bt->stream));
@@ -133,7 +135,7 @@ extern "C" int xs_batch_create(xs_batch **out, int nsys, const int *sys_ptr, con
     xs_batch_destroy(bt);
     return rc;
   }
-  BT_CHK(hipMemset(bt->bad, 0x7f, sizeof(int)));
+  BT_CHK(hipMemsetAsync(bt->bad, 0x7f, sizeof(int), bt->stream));
   xs_batch_prep(bt->stream, n, bt->rp, bt->ci, bt->v, bt->dinv, bt->dinv32, bt->v32, bt->bad);
   int bad = 0;
   BT_CHK(hipMemcpyAsync(&bad, bt->bad, sizeof(int), hipMemcpyDeviceToHost, bt->stream));
