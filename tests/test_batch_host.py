@@ -33,3 +33,17 @@ def test_flags_cleared_before_the_kernels_that_set_them(create, late):
     assert create(late, 6) == (xsolver_amd.XS_OK, 0, 1)    # slots would drop an entry
     assert create(late, 27) == (xsolver_amd.XS_OK, 0, 1)
     assert create(late, 5, bad_row=1200)[0] == xsolver_amd.XS_ERR_PIVOT
+
+
+def test_batch_that_fits_without_slots_is_taken(create):
+    """Diagonal slots are a second copy of the matrix: where the memory does
+    not hold them, the batch runs from its CSR arrays."""
+    lo, hi = 0, 1 << 22   # the memory that a batch without slots needs
+    while hi - lo > 1:
+        mid = (lo + hi) // 2
+        lo, hi = (lo, mid) if create(0, 6, memory=mid)[0] == xsolver_amd.XS_OK else (mid, hi)
+    assert create(0, 6, memory=lo)[0] == xsolver_amd.XS_ERR_MEMORY
+    assert create(0, 5, memory=hi) == (xsolver_amd.XS_OK, 0, 1)
+    # room for the FP64 slots (40 bytes a row) but not the FP32 ones as well
+    assert create(0, 5, memory=hi + 45 * 3000) == (xsolver_amd.XS_OK, 0, 1)
+    assert create(0, 5, memory=hi + 60 * 3000) == (xsolver_amd.XS_OK, 1, 0)

@@ -122,13 +122,13 @@ extern "C" int xs_batch_create(xs_batch **out, int nsys, const int *sys_ptr, con
   BT_CHK(hipMemcpyAsync(stat, bt->bad, sizeof(stat), hipMemcpyDeviceToHost, bt->stream));
   BT_CHK(hipStreamSynchronize(bt->stream));
   if (!stat[1] && stat[0] <= BT_RES_ND && bt->resrows) {
-    if ((rc = bt_alloc(&bt->dv, (size_t)BT_RES_ND * n)) ||
-        (rc = bt_alloc(&bt->dv32, (size_t)BT_RES_ND * n))) {
-      xs_batch_destroy(bt);
-      return rc;
+    if (bt_alloc(&bt->dv, (size_t)BT_RES_ND * n) || bt_alloc(&bt->dv32, (size_t)BT_RES_ND * n)) {
+      if (bt->dv) (void)hipFree(bt->dv);   // the CSR arrays are there and serve as well
+      bt->dv = nullptr;
+    } else {
+      xs_batch_dia(bt->stream, nsys, n, bt->sys_ptr, bt->off, bt->rp, bt->ci, bt->v, bt->dv,
+                   bt->dv32);
     }
-    xs_batch_dia(bt->stream, nsys, n, bt->sys_ptr, bt->off, bt->rp, bt->ci, bt->v, bt->dv,
-                 bt->dv32);
   }
   // the CSR values in FP32: only where a kernel reads them
   if ((!bt->dv || bt->nbig) && (rc = bt_alloc(&bt->v32, nnz))) {
