@@ -10,6 +10,7 @@
 #include <deque>
 #include <functional>
 
+#define __host__
 #define __device__
 #define __align__(n) __attribute__((aligned(n)))
 #define HIP_SYMBOL(x) (&x)

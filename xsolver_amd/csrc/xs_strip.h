@@ -18,14 +18,25 @@
 #define ST_IDLE (-2147483647 - 1)
 #define ST_STEP_SHIFT 14                                 // ring places fit below
 #define ST_MAX_STEPS ((1 << (31 - ST_STEP_SHIFT)) - 1)   // the last names no step
-#define ST_RING_MASK (ST_MAX_WAVES * ST_RING * 64 * 8 - 1)   // a place in bytes
-#define ST_SEQ_SHIFT 9                                   // its wave times four
-#define ST_SEQ_MASK ((ST_MAX_WAVES - 1) * 4)
+#define ST_SEQ_SHIFT 9                                   // a place's wave times four
 #define ST_LDS 4               // from this bit of carry's second: entries of the workgroup's other chains
 #define ST_MEM 8               // and entries read from memory
 #define ST_MAX_ROWS (1 << 28)  // 32-bit byte offsets
 static_assert(ST_RING * 64 == 1 << (ST_SEQ_SHIFT + 2) && ST_MAX_WAVES * ST_RING * 64 <= 1 << ST_STEP_SHIFT &&
               (ST_MAX_WAVES & (ST_MAX_WAVES - 1)) == 0, "code layout");
+
+// A code's ring place and the step counter of its wave as byte offsets into
+// the LDS arrays of a workgroup of W waves.  Codes that name no ring place
+// (their values are not used) give places in the arrays too: a step reads them
+// for all its lanes.
+template <int W>
+__host__ __device__ constexpr unsigned st_ring_byte(int code) {
+  return ((unsigned)code << 3) & (W * ST_RING * 64 * 8 - 1);
+}
+template <int W>
+__host__ __device__ constexpr unsigned st_seq_byte(int code) {
+  return ((unsigned)code >> ST_SEQ_SHIFT) & ((W - 1) * 4);
+}
 
 // One triangle.  Positions count along the solve (L: rows ascending, U:
 // descending).  Chain c owns the slots [cptr[c], cptr[c + 1]), a group of at

@@ -162,8 +162,8 @@ __global__ __launch_bounds__(W *XS_WAVE) void k_strip(const st_args S,
       bool ok = true;
       // (a code that names no ring place reads one all the same)
       auto take = [&](int cd, int &ps, double &v, int &f1, int &f2) {
-        lds_int *const sq = (lds_int *)((lds_char *)seq + ((unsigned)cd >> ST_SEQ_SHIFT & ST_SEQ_MASK));
-        lds_double *const rg = (lds_double *)((lds_char *)ring + ((unsigned)cd << 3 & ST_RING_MASK));
+        lds_int *const sq = (lds_int *)((lds_char *)seq + st_seq_byte<W>(cd));
+        lds_double *const rg = (lds_double *)((lds_char *)ring + st_ring_byte<W>(cd));
         ps = cd >> ST_STEP_SHIFT;
         f1 = *sq;
         v = *rg;
