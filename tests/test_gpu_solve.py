@@ -589,6 +589,36 @@ def test_update_values_then_solve(dev, precision):
     S.close()
 
 
+def test_update_values_behind_queued_work(dev):
+    """New values from a device tensor that the null stream is still busy
+    with: the formats that the context derives from them (the ELL copy and its
+    diagonal slots) are built after the copy has taken place."""
+    import torch
+    from xsolver_amd.autograd import solver_lib_update
+    A = gen.convdiff3d(48)
+    n, nnz = len(A[0]) - 1, len(A[2])
+    S = XSolver()
+    S.mat_setup(*A)
+    S.set_option("use_ell", 1)
+    x = torch.from_numpy(np.random.default_rng(3).uniform(-1, 1, n)).to(dev)
+    y1, yk = torch.empty_like(x), torch.empty_like(x)
+    v = torch.from_numpy(A[2]).to(dev)
+    big = torch.ones(1 << 27, dtype=torch.float64, device=dev)
+    st = torch.cuda.current_stream().cuda_stream
+    S.spmv(x, y1, st)
+    for k in range(1, 6):
+        w = v.clone()
+        torch.cuda.synchronize()
+        for _ in range(20):
+            big.mul_(1.0)              # ~10 ms of work ahead of the values
+        w.mul_(2.0 ** k)
+        solver_lib_update(S, w)
+        S.spmv(x, yk, st)
+        torch.cuda.synchronize()
+        assert torch.equal(yk, y1 * 2.0 ** k), k
+    S.close()
+
+
 def test_mixed_with_vector_csr(dev):
     """FP32 inner solve over the row-binned vector-CSR SpMV (FP32 kernel)."""
     A = gen.convdiff3d(24)

@@ -747,6 +747,9 @@ extern "C" int xs_mat_update_values(xs_ctx *c, const double *val, int on_device)
   if (!c->own_matrix) return XS_ERR_STATE;
   XS_HIP(hipMemcpy(c->A.v, val, sizeof(double) * c->A.nnz,
                    on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice));
+  // a copy between device buffers is not waited for, and the context's stream
+  // does not wait for the null stream
+  if (on_device) XS_HIP(hipStreamSynchronize(nullptr));
   if (c->use_ell) xs_build_ell(c->stream, c->A, c->ell.W, c->ell);
   if (c->have_At) xs_permute_vals(c->stream, c->A.nnz, c->perm_At, c->A.v, c->At.v);
   if (!c->pc_reuse) {   // else the factors of the earlier values stay
