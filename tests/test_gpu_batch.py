@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 
 import oracle
+import xsolver_amd
 from tests.helpers import X_TOL, say
 from xsolver_amd import XBatch, batch_concat, gen
 
@@ -129,3 +130,39 @@ def test_batch_resident_edges(dev, kind, sizes, precision):
         rc, x2, it2, rr2, _ = _noalloc(torch, dev, sys_ptr, rp, ci, v, b, 1e-9, 500)
         assert rc == 0 and np.array_equal(x2, x) and np.array_equal(it2, it)
         assert np.array_equal(rr2, rr)
+
+
+@pytest.mark.parametrize("precision", [0, 1], ids=["fp64", "fp32"])
+@pytest.mark.parametrize("value", [float("nan"), float("inf"), 1e200], ids=["nan", "inf", "overflow"])
+def test_batch_nonfinite_residual_is_not_converged(dev, value, precision):
+    """A right-hand side with a NaN or an infinity, or one whose norm overflows
+    (the base of relres is then infinite), in a system of each kernel and form:
+    its relres is NaN and the batch has not converged; the others get what they
+    get without it."""
+    import torch
+    rng = np.random.default_rng(12)
+    for kind in ("dia", "wide"):
+        sizes = (300, 513, 4097, 25600, 25601, 25700)   # the last two: k_batch_cg
+        sys_ptr, rp, ci, v = batch_concat([_band_system(n, kind, rng) for n in sizes])
+        b = gen.spmv((rp, ci, v), rng.uniform(-1, 1, int(sys_ptr[-1])))
+        bad = b.copy()
+        for s in (1, 3, 4):
+            bad[sys_ptr[s] + 7] = value
+        say(f"[batch nonfinite] {kind} {value} precision={precision}")
+        B = XBatch(sys_ptr, rp, ci, v)
+        x0, st0 = B.solve(b, tol=1e-9, maxiter=500, precision=precision)
+        it0, rr0 = B.results()
+        x1, st1 = B.solve(bad, tol=1e-9, maxiter=500, precision=precision)
+        it1, rr1 = B.results()
+        B.close()
+        assert st0 == 0 and st1 == xsolver_amd.XS_NOT_CONVERGED
+        for s, (lo, hi) in enumerate(zip(sys_ptr[:-1], sys_ptr[1:])):
+            if s in (1, 3, 4):
+                assert np.isnan(rr1[s]), (s, rr1[s])
+            else:
+                assert rr1[s] == rr0[s] and it1[s] == it0[s]
+                assert np.array_equal(x1[lo:hi], x0[lo:hi])
+        if precision == 0:
+            from tests.test_zz_no_alloc import _noalloc
+            rc, _, _, rr2, _ = _noalloc(torch, dev, sys_ptr, rp, ci, v, bad, 1e-9, 500)
+            assert rc == 0 and np.array_equal(np.isnan(rr2), np.isnan(rr1))

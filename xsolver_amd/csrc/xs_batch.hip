@@ -221,6 +221,13 @@ __device__ int bt_pattern_ok(int r0, int r1, int N, int nnz, const int *__restri
   return bad == 0.0;
 }
 
+// ||r|| / ||b - A x0|| from the squares; NaN when the base is not finite (a
+// NaN or an infinity in b, x0 or A, or a norm that overflows): such a system
+// has no residual to speak of and has not converged
+__device__ __forceinline__ double bt_relres(double rn, double bb) {
+  return isfinite(bb) ? (bb > 0.0 ? sqrt(rn / bb) : 0.0) : __builtin_nan("");
+}
+
 // One system on rows [r0, r1): FP64 CG from x0 (PREC 0), or FP32 CG with
 // FP64 reliable updates (PREC 1).
 #define BT_W 6   // row window of the SpMV (FP64: the register budget of 1024-thread groups)
@@ -255,7 +262,7 @@ __device__ void bt_system(int r0, int r1, int N, const int *__restrict__ rp,
       rn += t * t;
     });
     bt_sum2(rn, dm, red);
-    rel = bb > 0.0 ? sqrt(rn / bb) : 0.0;
+    rel = bt_relres(rn, bb);
   } else {
     // One FP32 CG recurrence (FP32 values, vectors and SpMV) with reliable
     // updates: whenever its residual has dropped by inner_tol since the last
@@ -273,7 +280,8 @@ __device__ void bt_system(int r0, int r1, int N, const int *__restrict__ rp,
     });
     bt_sum2(rn64, dm, red);
     const double bb = rn64;   // ||b - A x0||^2: the base of tol and relres
-    if (!(bb > 0.0)) return;  // x0 solves the system
+    rel = bt_relres(bb, bb);
+    if (!isfinite(bb) || bb == 0.0) return;  // nothing to solve for, or x0 solves it (rel 0)
     double rref = sqrt(bb), tau = 0.0, t2 = 0.0;
     for (int i = r0 + threadIdx.x; i < r1; i += BT_THREADS) {
       const float ri = r[i], zi = dinv32[i] * ri;
@@ -637,7 +645,8 @@ __device__ void rs_system(const M &A, const M64 &A64, int m, const T *__restrict
   };
   residual(true);
   const double bb = rn;   // the base of tol and relres
-  if (PREC == 1 ? !(bb > 0.0) : bb == 0.0) return;   // x0 solves the system
+  rel = bt_relres(bb, bb);
+  if ((PREC == 1 && !isfinite(bb)) || bb == 0.0) return;   // nothing to solve for, or x0 solves it (rel 0)
   const double res0 = sqrt(bb);
   double rref = res0;     // PREC 1: the last FP64 residual
   bool fresh = true;      // PREC 1: x and rel hold it
@@ -736,7 +745,7 @@ __device__ void rs_system(const M &A, const M64 &A64, int m, const T *__restrict
   });
   __syncthreads();
   residual(false);
-  rel = sqrt(rn / bb);
+  rel = bt_relres(rn, bb);
 }
 
 // Systems of at most BT_RES_ROWS rows, from the queue.  ND: BT_RES_ND
