@@ -619,3 +619,47 @@ def test_trsv_chains_edges(dev, name):
     assert rel_err(out[1][0], oracle.lower_solve(L, b)) < 6.2e-14
     assert rel_err(out[1][1], oracle.upper_solve(U, dinv, b)) < 6.2e-14
     assert rel_err(out[1][2], out[0][2]) < 6 * 6.2e-14
+
+
+@pytest.mark.parametrize("name", ["one_narrow", "four", "planes"])
+def test_captured_exact_apply_follows_setup(dev, name):
+    """An exact apply recorded into a graph solves with the factor of the last
+    set-up, whichever came first, and can be recorded right after one."""
+    import torch
+    from xsolver_amd.autograd import solver_lib_update
+    dims, offs, chains = CHAINS[name]
+    A = _grid_stencil(dims, offs, 12)
+    n = len(A[0]) - 1
+    say(f"[captured apply] {name} n={n}")
+    rng = np.random.default_rng(13)
+    b = dev_tensor(rng.uniform(-1, 1, n), dev)
+    y, ye = torch.empty_like(b), torch.empty_like(b)
+    S = XSolver()
+    S.mat_setup(*A)
+    S.pc_settype("ilu0")
+    S.set_option("parilu_async", 0)
+    S.pc_setup()
+    S.pc_apply(b, ye, torch_stream())   # the pattern's chains
+    torch.cuda.synchronize()
+    assert S.time_ms("trsv:chains") == chains
+
+    def record():
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            S.pc_apply(b, y, torch_stream())
+        return g
+
+    graph = record()
+    for step in range(3):
+        if step:
+            solver_lib_update(S, dev_tensor(A[2] * (1.0 + 0.3 * rng.uniform(size=len(A[2]))), dev))
+            S.pc_setup()
+        if step == 2:
+            graph = record()
+        y.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        S.pc_apply(b, ye, torch_stream())
+        torch.cuda.synchronize()
+        assert torch.equal(y, ye), step
+    S.close()

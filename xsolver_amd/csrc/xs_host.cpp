@@ -1615,6 +1615,15 @@ extern "C" int xs_pc_setup(xs_ctx *c) {
     default:
       return XS_ERR_STATE;
   }
+  // chains of the factor's pattern hold its values in their own order; they
+  // follow here, so that an apply recorded into a graph solves with the new
+  // ones and a later call has nothing left to do
+  xs_ilu &F = c->ilu;
+  for (xs_strip *S : {&F.sl, &F.su, &F.tsl, &F.tsu}) S->vals = false;
+  if (rc == XS_OK && F.chains && F.sl.ready && F.su.ready) {
+    xs_strip_values(c->stream, F.lu, F.sl);
+    xs_strip_values(c->stream, F.lu, F.su);
+  }
   XS_HIP(hipEventRecord(c->ev1, c->stream));
   XS_HIP(hipEventSynchronize(c->ev1));
   float ms = 0;
@@ -1622,8 +1631,7 @@ extern "C" int xs_pc_setup(xs_ctx *c) {
   c->t_pc_ms = ms;
   if (xs_take_launch_guard()) rc = XS_ERR_STATE;
   if (rc == XS_OK) c->pc_ready = true;
-  c->ilu.have_t = false;
-  for (xs_strip *S : {&c->ilu.sl, &c->ilu.su, &c->ilu.tsl, &c->ilu.tsu}) S->vals = false;
+  F.have_t = false;
   c->mixed_ready = false;   // FP32 copies of A and of the factors are rebuilt
   c->tell_ready = c->tell32_ready = false;   // and the sweep copies of the factors
   return rc;
