@@ -134,3 +134,53 @@ def test_autotune_triangular_solves_and_spmm(dev, tmp_path, monkeypatch):
             T.time_ms("tune:trsv_prog")) == (wg, ga, pr)
     assert len([l for l in cache.read_text().split("\n") if l.strip()]) == 2
     T.close()
+
+
+def _chain_factor(**opts):
+    """5-point factor whose triangular solves have 4 chains, on a 256 x 300 grid."""
+    kap = np.exp(0.3 * np.random.default_rng(3).standard_normal((300, 256)))
+    A = gen.vardiff2d(kap)
+    S = XSolver()
+    S.mat_setup(*A)
+    S.pc_settype("ilu0")
+    S.set_option("parilu_async", 0)
+    for k, v in opts.items():
+        S.set_option(k, v)
+    S.pc_setup()
+    return S, A
+
+
+def _solves(S, b, dev):
+    """L, U and transposed solves with the present factor."""
+    import torch
+    st = torch.cuda.current_stream().cuda_stream
+    out = [torch.empty_like(b) for _ in range(3)]
+    S.trsv(0, b, out[0], st)
+    S.trsv(1, b, out[1], st)
+    S.pc_apply_t(b, out[2], st)
+    torch.cuda.synchronize()
+    return out
+
+
+def _refactor(S, A, dev):
+    import torch
+    from xsolver_amd.autograd import solver_lib_update
+    solver_lib_update(S, torch.from_numpy(A[2]).to(dev))
+    S.pc_setup()
+
+
+def test_gather_width_leaves_the_chains(dev):
+    """The gather width is the general solve's: a factor with chains keeps them
+    over it and over a set-up with new values."""
+    import torch
+    S, A = _chain_factor()
+    b = torch.ones(len(A[0]) - 1, dtype=torch.float64, device=dev)
+    ref = _solves(S, b, dev)
+    assert S.time_ms("trsv:chains") == 4
+    for ga in (16, 4, 0):
+        S.set_option("trsv_gather", ga)
+        _refactor(S, A, dev)
+        out = _solves(S, b, dev)
+        assert S.time_ms("trsv:chains") == 4, ga
+        assert all(torch.equal(x, y) for x, y in zip(out, ref))
+    S.close()

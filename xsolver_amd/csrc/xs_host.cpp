@@ -1058,7 +1058,7 @@ static int build_strips(xs_ctx *c, int n, const int *rp, const int *ci, const in
 static int ensure_trsv_sched(xs_ctx *c, bool exact, int need) {
   xs_ilu &F = c->ilu;
   if (!exact && c->lsweeps >= 0 && c->usweeps >= 0) return XS_OK;
-  const bool chains = (need & NEED_CHAINS) && F.chains && F.trsv_prog != 1 && xs_ilu_gather(F) != 16;
+  const bool chains = (need & NEED_CHAINS) && xs_ilu_chains(F);
   auto need_groups = [&]() {
     return F.sched_pending && ((need & NEED_GROUPS) || !(chains && F.sl.ready));
   };
@@ -1620,7 +1620,7 @@ extern "C" int xs_pc_setup(xs_ctx *c) {
   // ones and a later call has nothing left to do
   xs_ilu &F = c->ilu;
   for (xs_strip *S : {&F.sl, &F.su, &F.tsl, &F.tsu}) S->vals = false;
-  if (rc == XS_OK && F.chains && F.sl.ready && F.su.ready) {
+  if (rc == XS_OK && xs_ilu_chains(F) && F.sl.ready && F.su.ready) {
     xs_strip_values(c->stream, F.lu, F.sl);
     xs_strip_values(c->stream, F.lu, F.su);
   }
@@ -2209,7 +2209,7 @@ int xs_build_factor_transpose(xs_ctx *c) {
   xs_ilu &F = c->ilu;
   if (F.have_t) return XS_OK;
   int rc;
-  const bool chains = F.chains && F.trsv_prog != 1 && xs_ilu_gather(F) != 16;
+  const bool chains = xs_ilu_chains(F);
   // a pattern stays as it is over new values; what its solves need is built
   // again when the options ask for the other form
   if (!F.have_tp || (chains ? !F.tsl.tried : F.tlgb == nullptr)) {
