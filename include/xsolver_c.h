@@ -216,13 +216,14 @@ int xs_set_option(xs_ctx *ctx, const char *name, double value);
  * 50%, with the k-RHS SpMM's 2 or 4 columns per thread timed at k = 16), and
  * keeps the fastest.  Called after xs_pc_setup with an ILU-type
  * preconditioner it also times the exact triangular solves over persistent
- * workgroups 128..1024, gather widths 4 / 16 and both group modes and keeps
- * the fastest.  With the environment variable XS_TUNE_CACHE naming a file,
+ * workgroups 128..1024, gather widths 4 / 16 and both group modes, and over
+ * the factor's chains where it has them (option trsv_chains), and keeps the
+ * fastest.  With the environment variable XS_TUNE_CACHE naming a file,
  * results are read from and appended to it per matrix (and factor)
  * signature.  Choices and times are queried with xs_get_time_ms("tune:chunk"
  * | "tune:ell" | "tune:us" | "tune:vec_lanes" | "tune:long_thr" |
  * "tune:spmm_cw" | "tune:trsv_wg" | "tune:trsv_gather" | "tune:trsv_prog" |
- * "tune:trsv_us"; -1 when not tuned).  The SpMV kernel in
+ * "tune:trsv_chains" | "tune:trsv_us"; -1 when not tuned).  The SpMV kernel in
  * use: xs_get_time_ms("spmv:kernel") = 0 LDS row blocks, 1 vector CSR, 2 ELL;
  * xs_get_time_ms("spmv:idx16") = 1 when the ELL copy stores 16-bit column
  * offsets (every entry within 32767 of its row), 0 when it reads int32

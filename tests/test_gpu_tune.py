@@ -9,6 +9,7 @@ import pytest
 
 import oracle
 from tests.helpers import random_sparse, say, true_relres
+from tests.test_gpu_kernels import S5, _grid_stencil
 from xsolver_amd import XSolver, gen
 
 pytestmark = pytest.mark.gpu
@@ -137,9 +138,9 @@ def test_autotune_triangular_solves_and_spmm(dev, tmp_path, monkeypatch):
 
 
 def _chain_factor(**opts):
-    """5-point factor whose triangular solves have 4 chains, on a 256 x 300 grid."""
-    kap = np.exp(0.3 * np.random.default_rng(3).standard_normal((300, 256)))
-    A = gen.vardiff2d(kap)
+    """Dominant 5-point matrix on a 256 x 300 grid and its factor, whose
+    triangular solves have 4 chains."""
+    A = _grid_stencil((256, 300), S5, 11)
     S = XSolver()
     S.mat_setup(*A)
     S.pc_settype("ilu0")
@@ -183,4 +184,52 @@ def test_gather_width_leaves_the_chains(dev):
         out = _solves(S, b, dev)
         assert S.time_ms("trsv:chains") == 4, ga
         assert all(torch.equal(x, y) for x, y in zip(out, ref))
+    S.close()
+
+
+def test_tuned_chains_stay_chosen(dev, tmp_path, monkeypatch):
+    """A factor with chains: the tuner's choice between them and the general
+    solve, either way (the cached line edited), holds over a set-up with new
+    values, for the transposed solves, and in a context that reads the cache;
+    a context that rules chains out has a line of its own."""
+    import torch
+    cache = tmp_path / "tune.txt"
+    monkeypatch.setenv("XS_TUNE_CACHE", str(cache))
+    S, A = _chain_factor()
+    b = torch.from_numpy(np.random.default_rng(5).uniform(-1, 1, len(A[0]) - 1)).to(dev)
+    ref = _solves(S, b, dev)
+    assert S.time_ms("tune:trsv_chains") == -1
+    S.autotune()
+    chosen, us = S.time_ms("tune:trsv_chains"), S.time_ms("tune:trsv_us")
+    say(f"[tune] 256 x 300: chains {chosen}, {us:.1f} us per lower + upper solve")
+    assert chosen in (0, 1) and us > 0
+    S.close()
+    lines = cache.read_text().splitlines()
+    assert len(lines) == 2 and lines[1].startswith("trsv+chains:")
+    f = lines[1].split()
+    # key, workgroups, gather, group mode, chains, us
+    assert len(f) == 6 and f[4] == str(int(chosen))
+    for pr, ch in (("0", "1"), ("1", "1"), ("0", "0"), ("1", "0")):
+        f[2:5] = ["16" if pr == "1" else "4", pr, ch]
+        cache.write_text(lines[0] + "\n" + " ".join(f) + "\n")
+        S, _ = _chain_factor()
+        _solves(S, b, dev)   # (chains of both are there before the tuner decides)
+        S.autotune()
+        assert S.time_ms("tune:trsv_chains") == int(ch)
+        for rep in range(2):
+            out = _solves(S, b, dev)
+            assert S.time_ms("trsv:chains") == (4 if ch == "1" else 0), (pr, ch, rep)
+            for x, y in zip(out, ref):
+                # (the general solve: the bound of test_trsv_chains_edges)
+                assert torch.equal(x, y) if ch == "1" else \
+                    (x - y).abs().max() <= 6 * 6.2e-14 * y.abs().max(), (pr, ch, rep)
+            _refactor(S, A, dev)
+        S.close()
+    assert len(cache.read_text().splitlines()) == 2
+    S, _ = _chain_factor(trsv_chains=0)
+    S.autotune()
+    assert S.time_ms("tune:trsv_chains") == 0
+    assert cache.read_text().splitlines()[2].startswith("trsv:")
+    _solves(S, b, dev)
+    assert S.time_ms("trsv:chains") in (0, -1)
     S.close()

@@ -80,7 +80,7 @@ static void free_precond(xs_ctx *c) {
   for (xs_strip *S : {&F.sl, &F.su, &F.tsl, &F.tsu}) xs_strip_free(*S);
   c->tell_ready = c->tell32_ready = false;
   F = xs_ilu();
-  F.chains = c->trsv_chains;
+  F.chains = xs_ctx_chains(c);
   F.trsv_wg = c->trsv_wg;
   F.trsv_prog = c->trsv_prog;
   F.trsv_gather = c->trsv_gather;
@@ -445,9 +445,12 @@ static std::string shape_key(const char *kind, const int *hrp, int n, int nnz) {
 enum { NEED_CHAINS = 1, NEED_GROUPS = 2 };   // forms of the exact triangular solves
 static int ensure_trsv_sched(xs_ctx *c, bool exact, int need);
 
-// The triangular solves of a set-up factor: persistent workgroups, gather
-// width and group mode, each combination timed on a lower plus an upper
-// solve; the fastest is kept (and cached by the factor's shape).
+// The triangular solves of a set-up factor, each form timed on a lower plus an
+// upper solve: the general solve's persistent workgroups, gather width and
+// group mode in every combination (k-column and FP32 solves use the fastest
+// whatever comes next), then the chains where the factor has them, whose own
+// shape is fixed.  The choice is cached by the factor's shape and by whether
+// chains were a candidate.
 static int tune_trsv(xs_ctx *c) {
   int rc;
   if ((rc = ensure_trsv_sched(c, true, NEED_CHAINS | NEED_GROUPS))) return rc;
@@ -455,33 +458,51 @@ static int tune_trsv(xs_ctx *c) {
   std::vector<int> hrp(F.n + 1);
   XS_HIP(hipStreamSynchronize(c->stream));
   XS_HIP(hipMemcpy(hrp.data(), F.rp, sizeof(int) * (F.n + 1), hipMemcpyDeviceToHost));
-  const std::string key = shape_key("trsv", hrp.data(), F.n, F.nnz);
+  const bool chains = F.chains;
+  const std::string key = shape_key(chains ? "trsv+chains" : "trsv", hrp.data(), F.n, F.nnz);
   std::vector<double> tv;
-  int bwg = F.trsv_wg, bga = xs_ilu_gather(F), bpr = F.trsv_prog;
+  int bwg = F.trsv_wg, bga = xs_ilu_gather(F), bpr = F.trsv_prog, bch = 0;
   double bus = 0.0;
-  if (tune_cache_get(key, tv, 4)) {
-    bwg = (int)tv[0]; bga = (int)tv[1]; bpr = (int)tv[2]; bus = tv[3];
+  if (tune_cache_get(key, tv, 5)) {
+    bwg = (int)tv[0]; bga = (int)tv[1]; bpr = (int)tv[2]; bch = tv[3] != 0.0; bus = tv[4];
   } else {
-    double *b = xs_ctx_vec(c, 0), *x = xs_ctx_vec(c, 1);
+    struct keep_chains {   // the general solve while it is timed; restored on every path
+      xs_ilu &F;
+      bool on;
+      ~keep_chains() { F.chains = on; }
+    } kc{F, chains};
+    double *b = xs_ctx_vec(c, 0), *x = xs_ctx_vec(c, 1), us;
     XS_HIP(hipMemsetAsync(b, 0, sizeof(double) * c->A.n, c->stream));
     bus = 1e30;
     static const int wgs[] = {128, 256, 512, 1024}, gathers[] = {4, 16};
+    F.chains = false;
     for (int wg : wgs)
       for (int ga : gathers)
         for (int pr = 0; pr < 2; ++pr) {
           F.trsv_wg = wg;
           F.trsv_gather = ga;
           F.trsv_prog = pr;
-          double us;
           if ((rc = time_trsv(c, b, x, 3, &us))) return rc;
           if (us < bus) { bus = us; bwg = wg; bga = ga; bpr = pr; }
         }
-    tune_cache_put(key, {(double)bwg, (double)bga, (double)bpr, bus});
+    F.chains = chains;
+    if (xs_strip_used(F, F.sl)) {
+      if ((rc = time_trsv(c, b, x, 3, &us))) return rc;
+      if (us < bus) { bus = us; bch = 1; }
+    }
+    tune_cache_put(key, {(double)bwg, (double)bga, (double)bpr, (double)bch, bus});
   }
   c->trsv_wg = F.trsv_wg = bwg;
   c->trsv_gather = F.trsv_gather = bga;
   c->trsv_prog = F.trsv_prog = bpr;
+  // (a factor that has no chains leaves them allowed)
+  if (chains && F.sl.ready) {
+    c->trsv_chains = bch != 0;
+    F.chains = xs_ctx_chains(c);
+  }
+  F.have_t = false;   // the transposed solves need what the chosen form needs
   c->tune_trsv_us = bus;
+  c->tune_chains = bch != 0;
   return XS_OK;
 }
 
@@ -859,13 +880,15 @@ extern "C" int xs_set_option(xs_ctx *c, const char *name, double value) {
   }
   else if (k == "trsv_chains") {   // 1: FP64 solves of narrow factors over chains of groups
     c->trsv_chains = value != 0;
-    c->ilu.chains = c->trsv_chains;
+    c->ilu.chains = xs_ctx_chains(c);
     c->ilu.have_t = false;
   }
   else if (k == "trsv_progressive") {   // -1 auto, 0 scan chain groups, 1 lane by lane
     if (value < -1 || value > 1) return XS_ERR_ARG;
     c->trsv_prog = (int)value;
     c->ilu.trsv_prog = c->trsv_prog;
+    c->trsv_general = value == 1;
+    c->ilu.chains = xs_ctx_chains(c);
     c->ilu.have_t = false;
   }
   else if (k == "trsv_gather") {   // 0 by factor width, 4 or 16 off-group entries per poll
@@ -2098,6 +2121,7 @@ extern "C" double xs_get_time_ms(const xs_ctx *c, const char *phase) {
   if (!strcmp(phase, "tune:trsv_wg")) return c->tune_trsv_us > 0 ? c->trsv_wg : -1.0;
   if (!strcmp(phase, "tune:trsv_gather")) return c->tune_trsv_us > 0 ? c->trsv_gather : -1.0;
   if (!strcmp(phase, "tune:trsv_prog")) return c->tune_trsv_us > 0 ? c->trsv_prog : -1.0;
+  if (!strcmp(phase, "tune:trsv_chains")) return c->tune_trsv_us > 0 ? c->tune_chains : -1.0;
   if (!strcmp(phase, "tune:trsv_us")) return c->tune_trsv_us > 0 ? c->tune_trsv_us : -1.0;
   // SpMV kernel in use: 0 LDS row blocks, 1 vector CSR, 2 ELL
   if (!strcmp(phase, "spmv:kernel"))

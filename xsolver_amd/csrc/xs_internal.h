@@ -245,10 +245,10 @@ struct xs_ilu {
 };
 
 // the FP64 solves of one right-hand side run over chains where the factor has
-// them: asked for and not overruled, and the factor is narrow (chains have at
+// them: asked for (xs_ctx_chains), and the factor is narrow (chains have at
 // most ST_MAXQ + 1 entries per row; a wide one is not looked at)
 inline bool xs_ilu_chains(const xs_ilu &F) {
-  return F.chains && F.trsv_prog != 1 && xs_trsv_gather_width(F.nnz, F.n) != 16;
+  return F.chains && xs_trsv_gather_width(F.nnz, F.n) != 16;
 }
 // this triangle's solve does
 inline bool xs_strip_used(const xs_ilu &F, const xs_strip &S) {

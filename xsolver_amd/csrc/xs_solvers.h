@@ -49,10 +49,12 @@ struct xs_ctx {
   double tune_us = 0.0;
   int tune_L = 0, tune_long_thr = 0;  // vector-CSR lanes per row, long-row threshold
   double tune_trsv_us = 0.0;    // > 0 once the triangular solves are tuned
+  bool tune_chains = false;     // and their chains were the fastest
   bool fuse_p = false;          // BiCGSTAB forms p inside the first L pass (slower when launched directly)
   int use_graph = -1;           // replay batches as HIP graphs: 1 all solves, 0 none, -1 k-RHS blocks
   bool trsv_schedule = true;    // SpTRSV groups in dependency-level order
   bool trsv_chains = true;      // FP64 SpTRSV of narrow factors over chains of groups when possible
+  bool trsv_general = false;    // trsv_progressive = 1 was asked for: no chains
   int trsv_wg = 256;            // persistent workgroups of the SpTRSV
   int trsv_prog = -1;           // SpTRSV group mode (xs_tsched::prog), -1 = by factor width
   int trsv_gather = 0;          // SpTRSV gather width (4 or 16), 0 = by factor width
@@ -159,6 +161,10 @@ struct xs_ctx {
   std::vector<double> resvec;
   float t_pc_ms = 0.f, t_solve_ms = 0.f;
 };
+
+// the exact triangular solves may run over chains (options trsv_chains,
+// trsv_progressive)
+inline bool xs_ctx_chains(const xs_ctx *c) { return c->trsv_chains && !c->trsv_general; }
 
 int xs_ctx_ensure_work(xs_ctx *c, int nvec);
 
