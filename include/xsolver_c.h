@@ -189,7 +189,9 @@ int xs_pc_setilut(xs_ctx *ctx, double tol, int max_fill);
  *   "cg_resident"    1 (default) = CG with Jacobi or no preconditioner runs as
  *                    one launch when A has a diagonal-slot copy (spmv_dia) and
  *                    its rows and reach fit the chip; 0 = a launch per kernel.
- *                    Not used with use_graph = 0 or 1 or while "profile" is on
+ *                    Not used with use_graph = 0 or 1 or while "profile" is on.
+ *                    xs_get_time_ms("cg:resident") = workgroups of the last CG
+ *                    solve's launch, 0 = it took a launch per kernel
  *   "use_ell"        1 = ELL SpMV (same as advanced_pam[1] = 1)
  *   "spmv_dia"       1 (default) = when the ELL copy is built and the matrix
  *                    has at most 8 distinct column - row offsets (5- and

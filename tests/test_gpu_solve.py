@@ -676,6 +676,14 @@ CG_RES = {"tri1": lambda: _tridiag(1), "tri512": lambda: _tridiag(512),
           "poisson3d_37": lambda: gen.convdiff3d(37, pe=0.0)}
 
 
+def _cg_workgroups(n):
+    """Workgroups of the one-launch CG: one up to 4096 rows, then at most eight
+    with 2 or 4 rows a thread, then as many as 8 rows a thread take."""
+    if n <= 4096:
+        return 1
+    return next(g for r in (2, 4, 8) for g in [-(-n // (512 * r))] if g <= (8 if r < 8 else 256))
+
+
 @pytest.mark.parametrize("pc", ["jacobi", "none"])
 @pytest.mark.parametrize("name", list(CG_RES))
 def test_cg_one_launch_matches_kernel_loop(dev, name, pc):
@@ -698,7 +706,10 @@ def test_cg_one_launch_matches_kernel_loop(dev, name, pc):
         S.set_option("use_ell", 1)
         S.set_option("cg_resident", resident)
         assert S.time_ms("spmv:dia") > 0
+        assert S.time_ms("cg:resident") == -1
         x, st = S.solve(b, x0=x0)
+        # the path that ran: the fallback to the loop is silent
+        assert S.time_ms("cg:resident") == (_cg_workgroups(n) if resident else 0)
         runs = [(x, st, S.iterations, S.residual, S.initial_residual, S.resvec())]
         x, st = S.solve(np.zeros(n))                    # a zero residual
         runs.append((x, st, S.iterations, S.residual, S.initial_residual, S.resvec()))

@@ -24,6 +24,6 @@ struct xs_cgres_args {
 };
 // words of the exchange buffer for a system of n rows; 0: not for this kernel
 size_t xs_cgres_words(int n, int reach);
-// the whole solve; false when the system or the device does not allow it
-// (nothing has been launched that touches x)
-bool xs_cgres(hipStream_t s, const xs_cgres_args &A);
+// the whole solve: its workgroups, or 0 when the system or the device does
+// not allow it (nothing has been launched that touches x)
+int xs_cgres(hipStream_t s, const xs_cgres_args &A);

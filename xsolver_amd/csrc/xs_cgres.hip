@@ -311,18 +311,18 @@ static bool cr_launch(hipStream_t s, int G, const xs_cgres_args &A) {
   return true;
 }
 
-bool xs_cgres(hipStream_t s, const xs_cgres_args &A) {
+int xs_cgres(hipStream_t s, const xs_cgres_args &A) {
   int R, G;
   if (!(A.dv && A.b && A.x && A.st && A.slots && A.err && A.nd > 0 && A.nd <= XS_DIA_MAX) ||
       !cr_shape(A.n, A.reach, R, G))
-    return false;
+    return 0;
   if (G > 1) {
     const size_t len = CR_MAX_WG * 8 + 2 * (size_t)A.n;
     hipLaunchKernelGGL(k_cr_clear, dim3((unsigned)((len + 1023) / 1024)), dim3(256), 0, s, A.slots, len);
   }
 #define CR_M(ND, R_) (G > 1 ? cr_launch<ND, R_, true>(s, G, A) : cr_launch<ND, R_, false>(s, 1, A))
 #define CR_R(ND) (R == 2 ? CR_M(ND, 2) : R == 4 ? CR_M(ND, 4) : CR_M(ND, 8))
-  return A.nd <= 5 ? CR_R(5) : CR_R(XS_DIA_MAX);
+  return (A.nd <= 5 ? CR_R(5) : CR_R(XS_DIA_MAX)) ? G : 0;
 #undef CR_R
 #undef CR_M
 }

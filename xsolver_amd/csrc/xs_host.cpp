@@ -2129,6 +2129,8 @@ extern "C" double xs_get_time_ms(const xs_ctx *c, const char *phase) {
   // 1 when the ELL copy carries 16-bit column offsets
   if (!strcmp(phase, "spmv:idx16")) return c->ell.co ? 1.0 : 0.0;
   if (!strcmp(phase, "spmv:dia")) return (c->use_ell && c->ell.dv) ? (double)c->ell.nd : 0.0;
+  // workgroups of the last CG solve in one launch (0: a launch per kernel, -1: no CG solve yet)
+  if (!strcmp(phase, "cg:resident")) return (double)c->cg_wg;
   if (!strcmp(phase, "pc:dia")) return c->tell_ready ? (double)c->ilu.tl.nd : -1.0;
   if (!strcmp(phase, "parilu:dia")) return (double)c->ilu.pnd;
   // chains of L's exact solve (0: the general solve, -1: not looked at yet)

@@ -92,7 +92,8 @@ static int cg_resident(xs_ctx *c, const double *b, double *x, int *used) {
   A.err = c->counters;
   A.slots = c->cg_buf;
   A.z = c->cg_buf + 8 * CR_MAX_WG;
-  if (!xs_cgres(c->stream, A)) return XS_OK;
+  c->cg_wg = xs_cgres(c->stream, A);
+  if (!c->cg_wg) return XS_OK;
   *used = 1;
   XS_CHK(hipMemcpyAsync(c->h_state, c->st, sizeof(xs_state), hipMemcpyDeviceToHost, c->stream));
   XS_CHK(hipStreamSynchronize(c->stream));
@@ -101,6 +102,7 @@ static int cg_resident(xs_ctx *c, const double *b, double *x, int *used) {
 
 // Preconditioned CG, hip/Solver/xsolver_cg.cpp:16-74.
 int xs_solve_cg(xs_ctx *c, const double *b, double *x) {
+  c->cg_wg = 0;
   int used = 0, rc = cg_resident(c, b, x, &used);
   if (used) return rc;
   rc = xs_ctx_ensure_work(c, XS_NWORK);

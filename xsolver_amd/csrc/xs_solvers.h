@@ -108,6 +108,7 @@ struct xs_ctx {
   double *ts_partial = nullptr;
   unsigned long long *cg_buf = nullptr;   // exchange words of the one-launch CG
   size_t cg_words = 0;
+  int cg_wg = -1;                   // workgroups of the last CG solve, 0 = loop of kernels, -1 = none yet
   double *mdot_partial = nullptr;   // intel-family multi-dot partials
   size_t mdot_len = 0;
   size_t ts_partial_len = 0;
