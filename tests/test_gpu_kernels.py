@@ -511,11 +511,16 @@ def _rows_of_lengths(lens, n, seed):
     return np.array(rp, np.int32), np.concatenate(ci).astype(np.int32), np.concatenate(v)
 
 
+# the last rows of lengths: at the rule's edges, 40 and 256 entries and ten
+# times the mean, and at the rungs below which a lane sums a row
 @pytest.mark.parametrize("lens", [(1, 15, 16, 17), (16, 17, 63, 64, 65), (2, 2047, 3), (1500, 1, 1),
-                                  (17,)], ids=str)
+                                  (17,), (1,) * 30 + (40,), (1,) * 30 + (41,), (256, 1), (257, 1),
+                                  (6,) * 31 + (80,), (6,) * 31 + (90,),
+                                  (2,) * 20 + (48, 49, 96, 97, 192, 193, 300)],
+                         ids=lambda l: str(l) if len(l) < 8 else f"{len(l)}to{max(l)}")
 def test_csr_row_blocks_mixed_lengths(dev, lens):
     """Rows at the edges of the lane / wave split of the LDS row blocks
-    (XS_CSR_ROW_LANE entries), FP64 products and epilogues and the FP32 inner
+    (xs_csr_lane_rows, csr_limit), FP64 products and epilogues and the FP32 inner
     solve over the same blocks.  Bound: a row of m products summed in any order
     is within m eps sum |a x| of the exact sum, and so is the oracle's."""
     import torch
@@ -542,6 +547,44 @@ def test_csr_row_blocks_mixed_lengths(dev, lens):
         xs, st = S.solve(b)
         assert st == 0 and true_relres(A, b, xs) < 1e-10
     S.close()
+
+
+def test_csr_row_blocks_time_per_entry(dev):
+    """Rows a little past a limit of the lane / wave split cost about what
+    shorter ones do per entry (summed by a wave each, rows of 17 took 3.4 times
+    as long as rows of 16)."""
+    import torch
+    us = {}
+    for L in (16, 17, 27, 60, 100):
+        n = 3200000 // L
+        rng = np.random.default_rng(L)
+        # L ascending columns a row, about 40 apart, around the diagonal
+        c = np.arange(n)[:, None] + np.cumsum(rng.integers(1, 80, (n, L)), 1) - 20 * L
+        c = np.sort(np.clip(c, 0, None) % (n + 100 * L), 1).astype(np.int64)
+        keep = np.ones_like(c, bool)
+        keep[:, 1:] = c[:, 1:] != c[:, :-1]
+        keep &= c < n
+        rp = np.append(0, np.cumsum(keep.sum(1))).astype(np.int32)
+        ci = c[keep].astype(np.int32)
+        S = XSolver()
+        S.mat_setup(rp, ci, rng.uniform(-1, 1, len(ci)))
+        S.set_option("spmv_kernel", 0)
+        assert S.time_ms("spmv:kernel") == 0
+        x = torch.ones(n, dtype=torch.float64, device=dev)
+        y = torch.empty_like(x)
+        best = 1e30
+        for _ in range(6):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            for _ in range(20):
+                S.spmv(x, y, torch_stream())
+            b.record()
+            torch.cuda.synchronize()
+            best = min(best, 50e6 * a.elapsed_time(b) / len(ci))   # ps per entry
+        us[L] = best
+        S.close()
+    say("[csr time] ps per entry", {k: round(v, 1) for k, v in us.items()})
+    assert max(us.values()) < 2 * us[16], us
 
 
 def _grid_stencil(dims, offs, seed):

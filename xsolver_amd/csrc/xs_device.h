@@ -362,50 +362,67 @@ __device__ __forceinline__ void reduce_finish(double (&v)[NV], const xs_reduce &
 }
 
 // ---------------------------------------------------------------------------
-// LDS row blocks of the CSR SpMV (FP64 and FP32).  What bounded it: one
-// thread summed each row from LDS, and a block waited for its longest row --
-// a row of 2000 entries is a chain of 2000 LDS reads (262147 rows of 4 to
-// 2000 entries, 2.8e6 in all: 70 us, 0.55 TB/s).  Rows of more than
-// XS_CSR_ROW_LANE entries are summed by their wave instead.
+// LDS row blocks of the CSR SpMV (FP64 and FP32): the sums of a block's rows
+// from its staged products.  What bounded them: one thread summed each row,
+// and a block waited for its longest row -- a row of 2000 entries is a chain
+// of 2000 LDS reads (262147 rows of 4 to 2000 entries, 2.8e6 in all: 68 us,
+// 0.55 TB/s).  A wave takes 64 rows at a time, a lane each, and sums the long
+// ones among them one by one with all its lanes.
+//
+// Which are long: a wave's sum of a row takes as long as a lane's chain of
+// about XS_CSR_WIDE reads, so the limit is the rung of csr_limit at which the
+// longest chain below it and the sums above it take least; a matrix without
+// such rows is summed by lanes alone (xs_csr_lane_rows).  A lane reads four
+// entries ahead of its sum, whose order stays.  Measured, us: the 262147 rows
+// 68 -> 20.6; 4e6 entries in rows of 17 19.1 -> 18.6, of 100 22.6 -> 18.5, of
+// 1 to 199 29.0 -> 21.0, of 400 42.6 -> 19.3.  (Every row beyond 16 entries by
+// its wave, as tried: rows of 17 66, of 100 32.  The largest row instead of
+// the last rung, by a reduction over the wave: 2 to 3% slower throughout.)
 // ---------------------------------------------------------------------------
-#define XS_CSR_ROW_LANE 16
-// prod[k] = v[e0 + k] x[ci[e0 + k]], k < ne: four entries per thread and step,
-// their loads branch-free (past the end the last entry is read again) so that
-// all are issued before any wait
-template <class T>
-__device__ __forceinline__ void csr_stage(T *prod, int e0, int ne, const int *__restrict__ ci,
-                                          const T *__restrict__ v, const T *__restrict__ x) {
-  for (int k0 = threadIdx.x; k0 < ne; k0 += 4 * XS_BLOCK) {
-    int c[4];
-    T a[4];
+#define XS_CSR_WIDE 24
+// The rows of more entries than the result are summed by the wave; n: this
+// lane's row, wide: the ballot of the longer ones.
+__device__ __forceinline__ int csr_limit(int n, unsigned long long &wide) {
+  int best = 0, lim = 0;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int k = e0 + min(k0 + q * XS_BLOCK, ne - 1);
-      c[q] = ci[k];
-      a[q] = v[k];
+  for (int t : {16, 48, 96, 192}) {
+    const unsigned long long m = __ballot(n > t);
+    const int cost = t + XS_CSR_WIDE * __popcll(m);   // wave-uniform, as all here
+    if (lim == 0 || cost < best) {
+      best = cost;
+      lim = t;
+      wide = m;
     }
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const T p = a[q] * x[c[q]];
-      if (k0 + q * XS_BLOCK < ne) prod[k0 + q * XS_BLOCK] = p;
-    }
+    if (m == 0) break;
   }
+  return lim;
 }
 
-// f(row, sum of the row's products) for the rows [r0, r1) of a staged block:
-// a wave takes 64 rows at a time, a lane each; the rows longer than
-// XS_CSR_ROW_LANE among them are then summed one by one by the whole wave.
+// f(row, sum of the row's products) for the rows [r0, r1) of a staged block.
 // Which wave and lane calls f for a row depends on the pattern alone.
+// lane_rows: the matrix has no rows that gain (xs_csr_lane_rows), a lane each.
 template <class T, class F>
 __device__ __forceinline__ void csr_reduce_rows(const T *prod, int r0, int r1, int e0,
-                                                const int *__restrict__ rp, F &&f) {
+                                                const int *__restrict__ rp, int lane_rows, F &&f) {
+  if (lane_rows) {
+    for (int r = r0 + threadIdx.x; r < r1; r += XS_BLOCK) {
+      const int a = rp[r] - e0, b = rp[r + 1] - e0;
+      T s = 0;
+#pragma unroll 4
+      for (int k = a; k < b; ++k) s += prod[k];
+      f(r, s);
+    }
+    return;
+  }
   const int lane = threadIdx.x & (XS_WAVE - 1);
   for (int b = r0 + (int)(threadIdx.x / XS_WAVE) * XS_WAVE; b < r1; b += XS_BLOCK) {
     const int r = b + lane;
     const int a = r < r1 ? rp[r] - e0 : 0, n = r < r1 ? rp[r + 1] - e0 - a : 0;
-    unsigned long long wide = __ballot(n > XS_CSR_ROW_LANE);
-    if (r < r1 && n <= XS_CSR_ROW_LANE) {
+    unsigned long long wide = 0;
+    const int lim = csr_limit(n, wide);
+    if (r < r1 && n <= lim) {
       T s = 0;
+#pragma unroll 4
       for (int k = a; k < a + n; ++k) s += prod[k];
       f(r, s);
     }

@@ -78,11 +78,24 @@ struct xs_spmv_plan {   // row blocks for the LDS-staged CSR kernel
   int nblk = 0;
   int chunk = 0;        // nnz budget per block
   int *blk_row = nullptr;  // [nblk + 1]
+  int lane_rows = 0;    // xs_csr_lane_rows of the matrix (0: not known)
   // row-binned vector CSR (used when vec != 0): rows of length <= long_thr
   // by groups of vec_L lanes, the nlong longer rows one wavefront each
   int vec = 0, vec_L = 0, long_thr = 0, nlong = 0;
   int *long_rows = nullptr;
 };
+
+// Whether a lane sums every row of an LDS row block.  A wave's sums of the
+// long ones pay off where a lane's chain is what a block waits for: rows of
+// more than 256 entries, or a few rows that are far longer than the others.
+// Elsewhere looking for them costs 2 to 5%.  Lanes against waves, us for 3 to
+// 4e6 entries: rows of 100 18.5 and 19.0, of 250 22.0 and 23.9, of 300 23.4 and
+// 21.1, of 1 to 299 23.5 and 26.0, of 1 to 399 25.5 and 24.7; rows of 6 with
+// 10% of 100 25.2 and 25.8, with 3% of 100 27.4 and 25.5, with 1% of 100 26.2
+// and 24.3, with 1% of 40 24.2 and 24.7.
+inline int xs_csr_lane_rows(int longest, double mean) {
+  return longest <= 256 && (longest <= 40 || longest <= 10.0 * mean);
+}
 
 // Diagonal slots: at most this many distinct column - row offsets in a matrix
 // (a 7-point stencil has 7) give its single-vector FP64 SpMV a copy without

@@ -68,7 +68,7 @@ template <int EPI>
 __global__ __launch_bounds__(XS_BLOCK) void k_spmv_csr(
     const int *__restrict__ rp, const int *__restrict__ ci, const double *__restrict__ v,
     const double *__restrict__ x, double *__restrict__ y, const int *__restrict__ blk_row,
-    const double *__restrict__ b, const double *__restrict__ w, xs_reduce R) {
+    const double *__restrict__ b, const double *__restrict__ w, int lane_rows, xs_reduce R) {
   __shared__ double prod[XS_SPMV_LDS];
   constexpr int NV = (EPI == EPI_DOT2) ? 2 : 1;
   constexpr bool RED = (EPI == EPI_DOT1 || EPI == EPI_DOT2 || EPI == EPI_BMAXN);
@@ -81,9 +81,9 @@ __global__ __launch_bounds__(XS_BLOCK) void k_spmv_csr(
     const int e0 = rp[r0], e1 = rp[r1];
     const int ne = e1 - e0;
     if (ne <= XS_SPMV_LDS) {
-      csr_stage(prod, e0, ne, ci, v, x);
+      for (int k = threadIdx.x; k < ne; k += XS_BLOCK) prod[k] = v[e0 + k] * x[ci[e0 + k]];
       __syncthreads();
-      csr_reduce_rows(prod, r0, r1, e0, rp,
+      csr_reduce_rows(prod, r0, r1, e0, rp, lane_rows,
                       [&](int r, double t) { epilogue<EPI, NV>(r, t, y, b, w, acc); });
     } else {
       const int lane = threadIdx.x & (XS_WAVE - 1);
@@ -346,11 +346,11 @@ void xs_launch_spmv_csr(hipStream_t s, const xs_csr &A, const xs_spmv_plan &P,
   }
   dim3 grid(P.nblk), blk(XS_BLOCK);
   switch (epi) {
-    case EPI_Y: hipLaunchKernelGGL(k_spmv_csr<EPI_Y>, grid, blk, 0, s, A.rp, A.ci, A.v, x, y, P.blk_row, b, w, R); break;
-    case EPI_BMAX: hipLaunchKernelGGL(k_spmv_csr<EPI_BMAX>, grid, blk, 0, s, A.rp, A.ci, A.v, x, y, P.blk_row, b, w, R); break;
-    case EPI_DOT1: hipLaunchKernelGGL(k_spmv_csr<EPI_DOT1>, grid, blk, 0, s, A.rp, A.ci, A.v, x, y, P.blk_row, b, w, R); break;
-    case EPI_DOT2: hipLaunchKernelGGL(k_spmv_csr<EPI_DOT2>, grid, blk, 0, s, A.rp, A.ci, A.v, x, y, P.blk_row, b, w, R); break;
-    case EPI_BMAXN: hipLaunchKernelGGL(k_spmv_csr<EPI_BMAXN>, grid, blk, 0, s, A.rp, A.ci, A.v, x, y, P.blk_row, b, w, R); break;
+    case EPI_Y: hipLaunchKernelGGL(k_spmv_csr<EPI_Y>, grid, blk, 0, s, A.rp, A.ci, A.v, x, y, P.blk_row, b, w, P.lane_rows, R); break;
+    case EPI_BMAX: hipLaunchKernelGGL(k_spmv_csr<EPI_BMAX>, grid, blk, 0, s, A.rp, A.ci, A.v, x, y, P.blk_row, b, w, P.lane_rows, R); break;
+    case EPI_DOT1: hipLaunchKernelGGL(k_spmv_csr<EPI_DOT1>, grid, blk, 0, s, A.rp, A.ci, A.v, x, y, P.blk_row, b, w, P.lane_rows, R); break;
+    case EPI_DOT2: hipLaunchKernelGGL(k_spmv_csr<EPI_DOT2>, grid, blk, 0, s, A.rp, A.ci, A.v, x, y, P.blk_row, b, w, P.lane_rows, R); break;
+    case EPI_BMAXN: hipLaunchKernelGGL(k_spmv_csr<EPI_BMAXN>, grid, blk, 0, s, A.rp, A.ci, A.v, x, y, P.blk_row, b, w, P.lane_rows, R); break;
   }
 }
 
