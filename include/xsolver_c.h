@@ -187,8 +187,9 @@ int xs_pc_setilut(xs_ctx *ctx, double tol, int max_fill);
  *                    rounded up to a power of two, long rows one wavefront
  *                    each).  0 and 1 also drop the automatic ELL copy.
  *   "cg_resident"    1 (default) = CG with Jacobi or no preconditioner runs as
- *                    one launch when A has a diagonal-slot copy (spmv_dia) and
- *                    its rows and reach fit the chip; 0 = a launch per kernel.
+ *                    one launch when A has a diagonal-slot copy (spmv_dia), its
+ *                    rows fit the chip and it reaches no farther than 5120 rows
+ *                    (past 4096 rows); 0 = a launch per kernel.
  *                    Not used with use_graph = 0 or 1 or while "profile" is on.
  *                    xs_get_time_ms("cg:resident") = workgroups of the last CG
  *                    solve's launch, 0 = it took a launch per kernel

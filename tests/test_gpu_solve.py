@@ -672,15 +672,20 @@ CG_RES = {"tri1": lambda: _tridiag(1), "tri512": lambda: _tridiag(512),
           "tri16385": lambda: _tridiag(16385), "tri36865": lambda: _tridiag(36865),
           "grid47x61": lambda: _grid2d(47, 61), "grid2000x3": lambda: _grid2d(2000, 3),
           "grid3x2000": lambda: _grid2d(3, 2000), "grid5000x9": lambda: _grid2d(5000, 9),
+          "grid5120x5": lambda: _grid2d(5120, 5), "grid5121x5": lambda: _grid2d(5121, 5),
           "grid191x193": lambda: _grid2d(191, 193), "poisson3d_12": lambda: gen.convdiff3d(12, pe=0.0),
           "poisson3d_37": lambda: gen.convdiff3d(37, pe=0.0)}
 
 
-def _cg_workgroups(n):
+def _cg_workgroups(A):
     """Workgroups of the one-launch CG: one up to 4096 rows, then at most eight
-    with 2 or 4 rows a thread, then as many as 8 rows a thread take."""
+    with 2 or 4 rows a thread, then as many as 8 rows a thread take; none where
+    the matrix reaches farther than 5120 rows."""
+    n = len(A[0]) - 1
     if n <= 4096:
         return 1
+    if np.abs(A[1] - np.repeat(np.arange(n), np.diff(A[0]))).max() > 5120:
+        return 0
     return next(g for r in (2, 4, 8) for g in [-(-n // (512 * r))] if g <= (8 if r < 8 else 256))
 
 
@@ -709,7 +714,7 @@ def test_cg_one_launch_matches_kernel_loop(dev, name, pc):
         assert S.time_ms("cg:resident") == -1
         x, st = S.solve(b, x0=x0)
         # the path that ran: the fallback to the loop is silent
-        assert S.time_ms("cg:resident") == (_cg_workgroups(n) if resident else 0)
+        assert S.time_ms("cg:resident") == (_cg_workgroups(A) if resident else 0)
         runs = [(x, st, S.iterations, S.residual, S.initial_residual, S.resvec())]
         x, st = S.solve(np.zeros(n))                    # a zero residual
         runs.append((x, st, S.iterations, S.residual, S.initial_residual, S.resvec()))

@@ -5,8 +5,10 @@
 // iteration whose work takes a fraction of a launch (256 x 256 rows, 5
 // points: 16.7 us per iteration, 14.5 of them inside kernels that move 4 MB
 // of cached data).  Measured against it, us per iteration: 33 x 33 rows 15.9
-// -> 2.5, 256 x 256 15.7 -> 5.8, 512 x 512 18.1 -> 7.7, 1000 x 1000 33 -> 16;
-// what is left are the two round trips between workgroups.  Here every workgroup owns a run of consecutive rows and
+// -> 2.5, 256 x 256 15.7 -> 5.8, 512 x 512 18.1 -> 7.7, 1000 x 1000 33 -> 16.
+// What is left is, in one workgroup, the barriers, reductions and divisions of
+// an iteration, and beyond that the two round trips between workgroups.  Here
+// every workgroup owns a run of consecutive rows and
 // keeps them for the whole solve: the matrix's diagonal slots, 1/a_ii, x, r
 // and q in registers (R rows per thread), p in LDS together with the p of the
 // rows within the matrix's reach on both sides (the halo).  Up to 512 R rows
@@ -269,16 +271,23 @@ __global__ void k_cr_clear(unsigned long long *p, size_t len) {
 // workgroups: 4.2).  Beyond, few workgroups: an exchange costs more the more
 // workgroups poll, local work little (us per iteration with R = 2 / 4 / 8:
 // 70^2 rows 4.0 / 4.1 / 4.7, 128^2 4.8 / 4.2 / 4.3, 256^2 6.6 / 6.0 / 5.8,
-// 512^2 13.3 / 9.4 / 7.7).
+// 512^2 13.3 / 9.4 / 7.7).  A thread polls for its halo rows one after another,
+// so a far reach costs what the launches do: the loop of kernels against one
+// launch, 37^3 rows 17.0 and 9.6, 48^3 17.1 and 12.1, 64^3 18.7 and 17.0, 70^3
+// (reach 4900) 22.3 and 21.5, 72^3 (5184) 22.7 and 22.9, 80^3 25.5 and 27.0,
+// 86^3 27.9 and 32.0; 5000 x 30 rows 18.1 and 16.9, 7000 x 40 19.9 and 23.0.
+#define CR_MAX_REACH (10 * CR_THREADS)   // 20 halo rows a thread
+static_assert((8 * CR_THREADS + 2 * CR_MAX_REACH) * sizeof(double) <= CR_LDS_MAX, "the window of p");
 static bool cr_shape(int n, int reach, int &R, int &G) {
   for (int r : {2, 4, 8})
     if (n <= r * CR_THREADS) { R = r; G = 1; return true; }
+  if (reach > CR_MAX_REACH) return false;
   for (int r : {2, 4, 8}) {
     const int g = (n + r * CR_THREADS - 1) / (r * CR_THREADS);
     if (g <= (r < 8 ? 8 : CR_MAX_WG)) {
       R = r;
       G = g;
-      return (size_t)(r * CR_THREADS + 2 * reach) * sizeof(double) <= CR_LDS_MAX;
+      return true;
     }
   }
   return false;
