@@ -614,6 +614,10 @@ CHAINS = {  # grid, stencil, chains of L (0: the general solve)
     "planes_carry": ((70, 12, 10), S7, 24),
     "three_entries": ((128, 9, 16), S9, 18),  # and a carry
     "own_ring": ((60, 9, 16), S9D, 9),        # another lane of the chain's last step
+    "three_blocks": ((130, 12, 10), S7, 36),
+    "four_blocks": ((200, 20, 20), S7, 0),    # fewer levels by the general solve
+    "four_blocks_one_row": ((193, 16, 16), S7, 64),   # which runs such groups together
+    "four_blocks_many_lines": ((198, 90, 8), S7, 360),
     "groups_too_short": ((12, 12, 12), S7, 0),
     "chains_too_short": ((40, 40, 5), S7, 0),
 }

@@ -382,6 +382,18 @@ __global__ __launch_bounds__(256) void k_strip_vals(size_t len, const int *__res
 // against 291).  A matrix without such a structure keeps k_trsv.
 #define ST_MIN_GROUP 16
 #define ST_MIN_CHAIN 8
+// On 3D grids whose lines are blocks of several groups, the chains of a line
+// fill half a workgroup or more, and a value passes through memory every line
+// or two; k_trsv has no more levels than lines, planes and blocks of a line.
+// Unless there are many lines, that is less (us, k_trsv against chains): 200 x
+// 20 x 20 48 and 52, 320 x 12 x 12 32 and 37, 256 x 40 x 40 91 and 95, 500 x 30
+// x 30 80 and 89, 320 x 64 x 64 147 and 157, 200 x 80 x 80 180 and 185; 256 x
+// 100 x 20 119 and 111, 200 x 128 x 50 196 and 179, 200^3 782 and 517; with
+// three blocks 130 x 20 x 20 47.3 and 46.9, 150 x 40 x 40 91 and 85, 160^3 423
+// and 330.  (It loses where a line ends in a group of one row, which it runs
+// together with the next line's: 257 x 40 x 40 169 and 101.)
+#define ST_LINE_BLOCKS 4
+#define ST_MIN_LINES 90
 // A workgroup of four chains has a SIMD for each; one of eight has half as many
 // places where a value goes through memory (about 2.5 us later) instead of
 // LDS.  512 x 512 grid (8 chains of 512 steps): 305 us by four, 343 by eight;
@@ -399,12 +411,19 @@ bool xs_strip_analyse(int n, const int *rp, const int *ci, const int *dpos, bool
     return upper ? n - 1 - ci[rp[r + 1] - 1 - t] : ci[rp[r] + t];
   };
   std::vector<int> grp(n);
+  int run = 0, blocks = 0;   // groups of this line of rows, of the longest
+  bool single = false;       // some group has one row
   for (int p = 0; p < n; ++p) {
     const int r = row(p), m = cnt(r);
     const bool chain = m > 0 && dep(r, m - 1) == p - 1;
     const int gs = P.gstart.empty() ? 0 : P.gstart.back();
     const bool first = P.gstart.empty() || !chain || p - gs == XS_WAVE;
-    if (first) P.gstart.push_back(p);
+    if (first) {
+      single |= p - gs == 1;
+      P.gstart.push_back(p);
+      run = chain ? run + 1 : 1;
+      blocks = std::max(blocks, run);
+    }
     // entries outside the group (the position before apart): few, and none
     // inside it
     const int ext = chain ? m - 1 : m;
@@ -453,6 +472,7 @@ bool xs_strip_analyse(int n, const int *rp, const int *ci, const int *dpos, bool
   }
   const int C = (int)len.size();
   if ((long)C * ST_MIN_CHAIN > G) return false;
+  if (P.Q >= 2 && blocks >= ST_LINE_BLOCKS && C < ST_MIN_LINES * blocks && !single) return false;
   // every dependency on another chain points to a lower one
   for (int p = 0; p < n; ++p) {
     const int r = row(p), m = cnt(r), c = P.gchain[grp[p]];
