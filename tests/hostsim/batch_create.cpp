@@ -26,7 +26,7 @@ void xs_batch_prep(hipStream_t s, int, const int *, const int *, const double *,
 }
 void xs_batch_prep64(hipStream_t, int, const int *, const int *, const double *, double *, unsigned *) {}
 void xs_batch_cg(hipStream_t, int, int, int, int, const xs_batch_args &) {}
-bool xs_batch_res(hipStream_t, int, int nsys, int, int, const xs_batch_args &P) {
+bool xs_batch_res(hipStream_t, int, int nsys, int, int, int, const xs_batch_args &P) {
   slots = P.dv != nullptr && P.dv32 != nullptr;
   v32 = P.v32 != nullptr;
   for (int q = 0; q < nsys; ++q) {

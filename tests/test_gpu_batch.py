@@ -166,3 +166,37 @@ def test_batch_nonfinite_residual_is_not_converged(dev, value, precision):
             from tests.test_zz_no_alloc import _noalloc
             rc, _, _, rr2, _ = _noalloc(torch, dev, sys_ptr, rp, ci, v, bad, 1e-9, 500)
             assert rc == 0 and np.array_equal(np.isnan(rr2), np.isnan(rr1))
+
+
+def test_noalloc_small_systems_launch(dev):
+    """A batch of mostly small systems runs in up to three launches of the
+    allocation-free entry: the same results bit for bit as with the sizes
+    known, each system solved by one of them, and a system whose columns leave
+    its block reported by one, whatever its size."""
+    import torch
+    from tests.test_zz_no_alloc import _noalloc
+    rng = np.random.default_rng(14)
+    sizes = [10] * 60 + [4095, 25601, 1, 4096, 4097, 25600] + [37] * 60
+    systems = [_band_system(n, "dia", rng) for n in sizes]
+    sys_ptr, rp, ci, v = batch_concat(systems)
+    n = int(sys_ptr[-1])
+    assert 4096 < n and n // len(sizes) <= 1024
+    b = gen.spmv((rp, ci, v), rng.uniform(-1, 1, n))
+    say(f"[noalloc small] {len(sizes)} systems, n={n}")
+    B = XBatch(sys_ptr, rp, ci, v)
+    x, st = B.solve(b, tol=1e-9, maxiter=500)
+    it, rr = B.results()
+    B.close()
+    assert st == 0
+    for rep in range(2):
+        rc, x2, it2, rr2, _ = _noalloc(torch, dev, sys_ptr, rp, ci, v, b, 1e-9, 500)
+        assert rc == 0 and np.array_equal(x2, x) and np.array_equal(it2, it)
+        assert np.array_equal(rr2, rr)
+    bad = np.array(ci)
+    off = [3, 60, 61, 64]   # 10, 4095, 25601 and 4097 rows
+    for s in off:
+        bad[rp[sys_ptr[s] + 1] - 1] = sys_ptr[s + 1]   # first row, into the next system
+    rc, x3, it3, rr3, _ = _noalloc(torch, dev, sys_ptr, rp, bad, v, b, 1e-9, 500)
+    ok = np.array([s not in off for s in range(len(sizes))])
+    assert rc == 0 and np.all(it3[~ok] == -1) and np.all(np.isnan(rr3[~ok]))
+    assert np.array_equal(it3[ok], it[ok]) and np.array_equal(rr3[ok], rr[ok])

@@ -8,6 +8,8 @@ void xs_batch_prep64(hipStream_t s, int n, const int *rp, const int *ci, const d
                      double *dinv, unsigned *queue);
 // rows of a system that k_batch_res can keep on one CU
 #define BT_RES_ROWS 25600
+// and in its form with two workgroups on a CU
+#define BT_RES_SMALL 4096
 // diagonal slots per row of its copy of the matrix: 5-point systems
 #define BT_RES_ND 5
 // N rows and nnz entries in the whole batch (N is the stride of the vectors
@@ -36,12 +38,12 @@ struct xs_batch_args {
   int *iters = nullptr;
   double *relres = nullptr;
 };
-// the systems of more than minrows rows / of at most BT_RES_ROWS rows
-// (maxrows: the largest of them that there can be); false: the launch was
-// refused
+// the systems of more than minrows rows (by k_batch_res: and at most maxrows, no
+// more than BT_RES_ROWS); false: the launch was refused.  Rows outside the
+// batch are reported by xs_batch_res with minrows = 0.
 void xs_batch_cg(hipStream_t s, int grid, int nsys, int minrows, int precision,
                  const xs_batch_args &P);
-bool xs_batch_res(hipStream_t s, int grid, int nsys, int maxrows, int precision,
+bool xs_batch_res(hipStream_t s, int grid, int nsys, int minrows, int maxrows, int precision,
                   const xs_batch_args &P);
 // diagonal slots: the offsets of every system (stat[0] = the most of one,
 // stat[1] = 1 when one has too many or unsorted rows; both 0 before), then

@@ -459,7 +459,8 @@ __global__ __launch_bounds__(BT_THREADS) void k_batch_cg(
 #define RS_RMAX 50                                   // rows per thread
 #define RS_LDS_K 39                                  // FP64: rows per thread whose p is in LDS
 #define RS_LDS_ROWS (RS_LDS_K * RS_THREADS)          // 19968 x 8 B = 156 KB of the CU's 160
-static_assert(BT_RES_ROWS == RS_RMAX * RS_THREADS, "capacity of the resident form");
+static_assert(BT_RES_ROWS == RS_RMAX * RS_THREADS && BT_RES_SMALL == 8 * RS_THREADS,
+              "capacity of the resident forms");
 
 // f(0), f(1), ..., f(N - 1) with constant arguments: loops over register
 // arrays that are unrolled whatever their size
@@ -748,13 +749,13 @@ __device__ void rs_system(const M &A, const M64 &A64, int m, const T *__restrict
   rel = bt_relres(rn, bb);
 }
 
-// Systems of at most BT_RES_ROWS rows, from the queue.  ND: BT_RES_ND
-// diagonal slots (xs_batch_dia), or 0 = CSR.  BIG = 0: at most 8 rows per
-// thread (4096 per system) with registers for two workgroups on a CU; 1: up
-// to RS_RMAX.
+// Systems of more than minrows and at most maxrows rows, from the queue.  ND:
+// BT_RES_ND diagonal slots (xs_batch_dia), or 0 = CSR.  BIG = 0: at most 8 rows
+// per thread (BT_RES_SMALL per system) with registers for two workgroups on a
+// CU; 1: up to RS_RMAX.
 template <int PREC, int ND, int BIG>
 __global__ __launch_bounds__(RS_THREADS, BIG ? 2 : 4) void k_batch_res(
-    int nsys, const xs_batch_args P) {
+    int nsys, int minrows, int maxrows, const xs_batch_args P) {
   typedef typename std::conditional<PREC == 0, double, float>::type T;
   extern __shared__ __align__(16) unsigned char rs_lds[];
   __shared__ double red[2][RS_WAVES][2];
@@ -770,8 +771,10 @@ __global__ __launch_bounds__(RS_THREADS, BIG ? 2 : 4) void k_batch_res(
     __syncthreads();
     if (sys < 0) break;
     const int r0 = P.sys_ptr[sys], r1 = P.sys_ptr[sys + 1], m = r1 - r0;
-    // larger systems are k_batch_cg's; rows outside the batch are reported here
-    if (m > BT_RES_ROWS && r0 >= 0 && r1 <= P.N) continue;
+    // the others' systems; rows outside the batch are reported by the launch
+    // with minrows = 0
+    const bool inside = r0 >= 0 && r1 <= P.N;
+    if (inside ? (m > maxrows || (minrows > 0 && m <= minrows)) : minrows > 0) continue;
     int it = 0;
     double rel = 0.0;
     if (ND == 0 && !bt_pattern_ok<RS_THREADS>(r0, r1, P.N, P.nnz, P.rp, P.ci, red[1])) {   // (the sums of rs_system start with red[0])
@@ -911,14 +914,14 @@ __global__ void k_batch_prep(int n, const int *__restrict__ rp, const int *__res
 }
 
 // FP64 Jacobi set-up only (1/a_ii; a zero or missing diagonal gives inf,
-// which the CG turns into a non-finite relres for that system), and the two
+// which the CG turns into a non-finite relres for that system), and the three
 // work-queue counters cleared by the same launch (thread 0), so a caller
 // under graph capture records kernels only.
 __global__ void k_batch_prep64(int n, const int *__restrict__ rp, const int *__restrict__ ci,
                                const double *__restrict__ v, double *__restrict__ dinv,
                                unsigned *queue) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < 2) queue[i] = 0u;
+  if (i < 3) queue[i] = 0u;
   if (i >= n) return;
   double d = 0.0;
   for (int e = rp[i]; e < rp[i + 1]; ++e)
@@ -946,28 +949,31 @@ static size_t res_lds(int maxrows, size_t es) {
 }
 
 template <int PREC, int ND, int BIG>
-static bool res_launch(hipStream_t s, int grid, int nsys, size_t lds, const xs_batch_args &P) {
+static bool res_launch(hipStream_t s, int grid, int nsys, int minrows, int maxrows, size_t lds,
+                       const xs_batch_args &P) {
   if (lds > 65536 &&
       hipFuncSetAttribute(reinterpret_cast<const void *>(&k_batch_res<PREC, ND, BIG>),
                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
     return false;
-  hipLaunchKernelGGL((k_batch_res<PREC, ND, BIG>), dim3(grid), dim3(RS_THREADS), lds, s, nsys, P);
+  hipLaunchKernelGGL((k_batch_res<PREC, ND, BIG>), dim3(grid), dim3(RS_THREADS), lds, s, nsys,
+                     minrows, maxrows, P);
   return true;
 }
 
 template <int PREC, int ND>
-static bool res_launch(hipStream_t s, int grid, int nsys, int maxrows, const xs_batch_args &P) {
+static bool res_launch(hipStream_t s, int grid, int nsys, int minrows, int maxrows,
+                       const xs_batch_args &P) {
   const size_t lds = res_lds(maxrows, PREC == 0 ? 8 : 4);
-  return maxrows <= 8 * RS_THREADS ? res_launch<PREC, ND, 0>(s, grid, nsys, lds, P)
-                                   : res_launch<PREC, ND, 1>(s, grid, nsys, lds, P);
+  return maxrows <= BT_RES_SMALL ? res_launch<PREC, ND, 0>(s, grid, nsys, minrows, maxrows, lds, P)
+                                 : res_launch<PREC, ND, 1>(s, grid, nsys, minrows, maxrows, lds, P);
 }
 
-bool xs_batch_res(hipStream_t s, int grid, int nsys, int maxrows, int precision,
+bool xs_batch_res(hipStream_t s, int grid, int nsys, int minrows, int maxrows, int precision,
                   const xs_batch_args &P) {
   if (nsys <= 0) return true;
   if (maxrows > BT_RES_ROWS) maxrows = BT_RES_ROWS;
-#define RS_GO(ND_) (precision == 0 ? res_launch<0, ND_>(s, grid, nsys, maxrows, P) \
-                                   : res_launch<1, ND_>(s, grid, nsys, maxrows, P))
+#define RS_GO(ND_) (precision == 0 ? res_launch<0, ND_>(s, grid, nsys, minrows, maxrows, P) \
+                                   : res_launch<1, ND_>(s, grid, nsys, minrows, maxrows, P))
   return P.dv ? RS_GO(BT_RES_ND) : RS_GO(0);
 #undef RS_GO
 }

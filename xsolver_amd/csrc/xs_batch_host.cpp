@@ -170,7 +170,7 @@ static int batch_run(xs_batch *bt, const double *d_b, double *d_x, double tol, i
   P.order = bt->order + bt->nbig;
   P.queue = bt->queue + 1;
   const int nres = bt->nsys - bt->nbig;
-  if (!xs_batch_res(s, std::min(nres, 2 * cus), nres, bt->resrows, precision, P))
+  if (!xs_batch_res(s, std::min(nres, 2 * cus), nres, 0, bt->resrows, precision, P))
     return XS_ERR_DEVICE;
   BT_CHK(hipGetLastError());
   BT_CHK(hipEventRecord(bt->e1, s));
@@ -224,6 +224,13 @@ extern "C" double xs_batch_get_time_ms(const xs_batch *bt) { return bt ? bt->ms 
 // ends.  Calls on one GPU share that GPU's array (the last call's contents
 // stay in it): calls that overlap on one GPU, on any streams, race.
 // ---------------------------------------------------------------------------
+// Mean rows up to which the small systems get a launch of their own.  The
+// device alone knows the sizes, and a batch of more than BT_RES_SMALL rows may
+// hold a large system, whose form leaves room for one workgroup on a CU:
+// 4096 systems of 4^2 to 16^2 rows 3.29 ms in that form, 1.45 in two launches
+// (k_batch_cg: 2.98); 1000 of 20^2 to 28^2 2.57 and 1.29; beyond, 200 of 16^2 to
+// 60^2 and 3 of 100^2, mean 1766: 12.6 and 14.0.
+#define NOALLOC_MEAN 1024
 #define XS_NOALLOC_HEADER 256   // bytes before the vectors: the queue counters
 static __device__ __align__(256) unsigned char
     scratch[XS_NOALLOC_HEADER + 7 * sizeof(double) * (size_t)XS_BATCH_NOALLOC_MAX_ROWS];
@@ -282,7 +289,13 @@ extern "C" int xs_batch_solve_noalloc(int nsys, int n, int nnz, const int *d_sys
   P.queue = queue; P.iters = d_iters; P.relres = d_relres;
   if (n > BT_RES_ROWS) xs_batch_cg(s, grid, nsys, BT_RES_ROWS, 0, P);
   P.queue = queue + 1;
-  if (!xs_batch_res(s, grid, nsys, std::min(n, BT_RES_ROWS), 0, P)) return XS_ERR_DEVICE;
+  // mostly small systems: theirs is the form with more of them on a CU
+  const int small = n > BT_RES_SMALL && n / nsys <= NOALLOC_MEAN ? BT_RES_SMALL : 0;
+  if (small) {
+    if (!xs_batch_res(s, grid, nsys, 0, small, 0, P)) return XS_ERR_DEVICE;
+    P.queue = queue + 2;
+  }
+  if (!xs_batch_res(s, grid, nsys, small, std::min(n, BT_RES_ROWS), 0, P)) return XS_ERR_DEVICE;
   if (hipGetLastError() != hipSuccess) return XS_ERR_DEVICE;
   return XS_OK;
 }
