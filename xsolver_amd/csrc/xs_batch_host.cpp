@@ -279,7 +279,7 @@ extern "C" int xs_batch_solve_noalloc(int nsys, int n, int nnz, const int *d_sys
   const int grid = std::min(nsys, 2 * cus);
   // one launch sets 1/a_ii and clears the queue counters (kernels only, so the
   // call can be captured into a graph); the sizes of the systems are on the
-  // device, so each of the two kernels passes over the other's
+  // device, so each of the launches passes over the others'
   xs_batch_prep64(s, n, d_rowptr, d_colidx, d_val, dinv, queue);
   xs_batch_args P;
   P.N = n; P.nnz = nnz;

@@ -334,7 +334,7 @@ __global__ __launch_bounds__(XS_BLOCK) void k_mspmm_ell(
   const int L = k / CW, per = XS_BLOCK / L;
   const int g = threadIdx.x % L, rl = threadIdx.x / L;
   // this thread's c-th column
-  auto jc = [&](int c) { return CW == 1 ? g : (c / 2) * 2 * L + 2 * g + (c & 1); };
+  auto jc = [&](int c) { return (c / 2) * 2 * L + 2 * g + (c & 1); };
   bool live[CW];
   bool any = false;
 #pragma unroll

@@ -39,10 +39,8 @@
 #include <algorithm>
 #include <unordered_map>
 
-#ifndef ST_STA
 #define ST_DEP 2     // steps ahead: values from memory
 #define ST_STA 8     // steps ahead: codes, factor values, b and 1/u_ii
-#endif
 #define ST_PACE 12   // steps ahead of the next chain
 
 struct st_args {
