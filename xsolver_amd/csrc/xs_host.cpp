@@ -230,10 +230,10 @@ static int make_vec(xs_ctx *c, const std::vector<int> &hrp, xs_spmv_plan &P, int
   P.long_thr = (long_mult ? long_mult : 8) * L;
   std::vector<int> lr;
   int mx = 0;
-  for (int i = 0; i < n; i++) {
-    mx = std::max(mx, hrp[i + 1] - hrp[i]);
-    if (hrp[i + 1] - hrp[i] > P.long_thr) lr.push_back(i);
-  }
+  for (int i = 0; i < n; i++) mx = std::max(mx, hrp[i + 1] - hrp[i]);
+  if (mx > P.long_thr)
+    for (int i = 0; i < n; i++)
+      if (hrp[i + 1] - hrp[i] > P.long_thr) lr.push_back(i);
   P.lane_rows = xs_csr_lane_rows(mx, avg);
   dfree(P.long_rows);
   P.nlong = (int)lr.size();
