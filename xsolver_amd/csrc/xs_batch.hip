@@ -443,7 +443,15 @@ __global__ __launch_bounds__(BT_THREADS) void k_batch_cg(
 // systems beyond 32 rows per thread).  512 systems of 32^2 to 160^2 rows:
 // FP64 63.5 -> 26.6 ms, FP32 40.4 -> 12.3 ms; the 160^2 system alone 99 -> 51
 // us per iteration (FP64), 66 -> 22 (FP32), now bound by the loads one CU has
-// in flight; 256 of 128^2 rows 119 -> 46 us (4.4 TB/s).
+// in flight; 256 of 128^2 rows 119 -> 46 us (4.45 TB/s).
+//
+// Batches in which some system has more than BT_RES_ND offsets, or rows that
+// do not ascend, are read from the CSR arrays (KB = 1: fewer loads in flight).
+// k_batch_cg against that form, ms: 512 7-point systems of 16^3 rows 3.13 and
+// 1.27 (FP32 2.11 and 1.21), 256 of 8^3 to 29^3 10.3 and 8.9 (6.4 and 6.3), 64 of
+// 20^3 to 29^3 8.5 and 8.3 (5.9 and 6.0), one of 29^3 6.0 and 6.1 (4.5 and 4.5);
+// 256 9-point systems of 32^2 to 160^2 18.1 and 13.7 (10.9 and 9.2); the 512
+// systems above with one 9-point system among them 85 and 68 (46 and 35).
 //
 // 512 threads with 256 registers each: the registers of a CU hold 512 KB
 // either way, and 8 waves that each have 20 loads in flight reach what one CU

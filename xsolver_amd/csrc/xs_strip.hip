@@ -18,10 +18,11 @@
 //    value is read from memory, where every row is also published;
 //  * only values from other workgroups go through memory, asked for two steps
 //    ahead; what does not depend on other rows is asked for eight steps ahead.
-// A step is then bound by its own instructions (about 200 at four cycles each
-// and an LDS round trip, 0.5 us), not by a memory access.  L of a 512 x 512
-// grid 421 -> 270 us, 1000 x 1000 871 -> 528, 64 x 64 56 -> 33; of a 7-point
-// grid 128^3 266 -> 234, 100^3 212 -> 187, 64^3 128 -> 96, 24^3 291 -> 37.
+// A step is then bound by its own instructions (178 of a wave by the counters,
+// 107 of them VALU, and an LDS round trip: 0.52 us), not by a memory access.  L
+// of a 512 x 512 grid 421 -> 270 us, 1000 x 1000 871 -> 526, 64 x 64 56 -> 33;
+// of a 7-point grid 128^3 262 -> 233, 100^3 210 -> 185, 64^3 129 -> 96, 24^3
+// 290 -> 37.
 // Chains depend on lower chains only (checked when the chains are formed) and
 // workgroups take them in that order by ticket, so the earliest unfinished
 // chain never waits: every wait ends.  Waits are bounded as in k_trsv.
@@ -394,8 +395,9 @@ __global__ __launch_bounds__(256) void k_strip_vals(size_t len, const int *__res
 #define ST_MIN_LINES 90
 // A workgroup of four chains has a SIMD for each; one of eight has half as many
 // places where a value goes through memory (about 2.5 us later) instead of
-// LDS.  512 x 512 grid (8 chains of 512 steps): 305 us by four, 343 by eight;
-// 128^3 (256 of 128): 294 and 256.
+// LDS.  L by four and by eight, us: 512 x 512 grid (8 chains of 512 steps) 270
+// and 294, 1000 x 1000 (16 of 1000) 526 and 581; 128^3 (256 of 128) 272 and
+// 233, 100^3 216 and 186, 64^3 103 and 96.
 #define ST_FOUR 4
 
 bool xs_strip_analyse(int n, const int *rp, const int *ci, const int *dpos, bool upper,
